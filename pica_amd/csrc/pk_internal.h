@@ -206,6 +206,24 @@ __device__ __forceinline__ int pk_select_bit(uint64_t m, int k)
     return pos;
 }
 
+// by one wavefront: pre[w] = set bits of mask[0 .. w), w <= words, 64 words at a time
+__device__ __forceinline__ void pk_mask_prefix(const uint64_t* mask, long* pre, int words, int lane)
+{
+    int run = 0;
+    for (int w0 = 0; w0 < words; w0 += 64) {
+        const int c = w0 + lane < words ? __popcll(mask[w0 + lane]) : 0;
+        int incl = c;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o);
+            if (lane >= o) incl += y;
+        }
+        if (w0 + lane < words) pre[w0 + lane] = run + incl - c;
+        run += __shfl(incl, 63);
+    }
+    if (lane == 0) pre[words] = run;
+}
+
 __device__ __forceinline__ void cell_coords(int c, const EnsGeom& eg, int cc[3])
 {
     const int q12 = (int)fastdiv((uint32_t)c, eg.div12), q2 = (int)fastdiv((uint32_t)c, eg.div2);
