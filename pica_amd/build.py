@@ -25,6 +25,7 @@ SOURCES = [
     ("pk_denoise.hip", ["-ffp-contract=fast"]),
     ("pk_project.hip", ["-ffp-contract=off"]),
     ("pk_snapshot.hip", ["-ffp-contract=off"]),
+    ("pk_transfer.hip", ["-ffp-contract=off"]),
 ]
 
 COMMON = [

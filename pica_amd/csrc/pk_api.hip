@@ -110,7 +110,8 @@ int pk_ctx_create(int device, pk_ctx** out)
     c->device = device;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipHostMalloc((void**)&c->flags_host, sizeof(int32_t) * PK_NFLAGS, hipHostMallocDefault) != hipSuccess ||
-        hipEventCreateWithFlags(&c->flags_ev, hipEventDisableTiming) != hipSuccess) {
+        hipEventCreateWithFlags(&c->flags_ev, hipEventDisableTiming) != hipSuccess ||
+        !(c->staging = pk_staging_create())) {
         if (c->flags_host) (void)hipHostFree(c->flags_host);
         if (c->stream) (void)hipStreamDestroy(c->stream);
         delete c;
@@ -139,6 +140,7 @@ void pk_ctx_destroy(pk_ctx* c)
     }
     for (auto ev : c->evpool) (void)hipEventDestroy(ev);
     if (c->flags_ev) (void)hipEventDestroy(c->flags_ev);
+    pk_staging_destroy(c->staging);
     if (c->flags_host) (void)hipHostFree(c->flags_host);
     (void)hipStreamDestroy(c->stream);
     delete c;
@@ -298,7 +300,7 @@ int pk_grid_copy(pk_grid* g, int comp, void* host, int dir)
     if (dir == PK_H2D)
         PK_HIP(c, hipMemcpyAsync(g->comp(comp), host, bytes, hipMemcpyHostToDevice, c->stream));
     else if (dir == PK_D2H)
-        PK_HIP(c, hipMemcpyAsync(host, g->comp(comp), bytes, hipMemcpyDeviceToHost, c->stream));
+        return pk_copy_to_host(c, host, g->comp(comp), bytes);
     else
         return pk_fail(c, PK_E_ARG, "pk_grid_copy: dir must be PK_H2D or PK_D2H");
     PK_HIP(c, hipStreamSynchronize(c->stream));

@@ -1545,7 +1545,7 @@ int pk_ens_download_impl(pk_ens* e, double* const* host, int64_t* off)
                            part_split(e, e->main), e->off, e->cnt, runstart.as<int64_t>(), of);
     PK_HIP(c, hipGetLastError());
     for (int k = 0; k < 7; k++)
-        if (host[k]) PK_HIP(c, hipMemcpyAsync(host[k], of.f[k], sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
+        if (host[k] && (r = pk_copy_to_host(c, host[k], of.f[k], sizeof(double) * n)) != PK_OK) return r;
     if (off)
         PK_HIP(c, hipMemcpyAsync(off, runstart.p, sizeof(int64_t) * (e->nsct + 1), hipMemcpyDeviceToHost, c->stream));
     PK_HIP(c, hipStreamSynchronize(c->stream));

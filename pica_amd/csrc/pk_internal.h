@@ -26,6 +26,8 @@ struct pk_timer_rec {
     long launches = 0;
 };
 
+struct pk_staging;
+
 struct pk_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -42,7 +44,12 @@ struct pk_ctx {
     int32_t* flags_host = nullptr;     // pinned, PK_NFLAGS
     hipEvent_t flags_ev = nullptr;     // recorded after a re-sort's flag copy (pk_ens_resort_begin)
     int opt[PK_OPT_N] = {PK_KERNEL_AUTO, 0, 3, 0};
+    pk_staging* staging = nullptr;     // pinned memory of copies to the host (pk_transfer.hip)
 };
+
+pk_staging* pk_staging_create();
+void pk_staging_destroy(pk_staging* s);
+int pk_copy_to_host(pk_ctx* c, void* host, const void* dev, size_t bytes);
 
 enum { PK_FLAG_ERR = 0, PK_FLAG_OVERFLOW = 1, PK_NFLAGS = 4 };
 
