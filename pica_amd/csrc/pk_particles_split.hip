@@ -31,12 +31,34 @@ namespace {
 
 constexpr int WAVES = PK_BLOCK / 64;
 constexpr int REC_WORDS = 8;     // deposit record: packed cell/shift/class, o[3], on[3], q w
-constexpr int QCAP = 256;        // change-queue records per workgroup
-// x-stride padding of the FP64 J tile (doubles).  With 8 x 8 x 8 nodes unpadded, the 4^3 cells a
-// wavefront's particles sit in fall on 8 of the 16 double-wide LDS bank pairs; +4 spreads them 4
-// per pair, which lowers the bank conflicts of the deposit atomics.
-constexpr int JPAD = 4;
-constexpr int IPAD = 4;          // x-stride padding of the field tile (floats), same purpose
+constexpr int QCAP = 192;        // change-queue records per workgroup
+
+// strides of the field tile (floats) and the J tile (doubles): of a component, an x plane, a y row
+struct TileStrides {
+    int itn, isx, isy, dtn, dsx, dsy;
+    int ni, nj;                  // floats of the field tile, doubles of the J tile
+};
+
+// The 64 cells of a 4^3 supercell are what a wavefront's 64 lanes hold (the interleave keeps them
+// so), and both tiles lay them on distinct LDS banks: the three components of a J row lie side by
+// side, 28 doubles a row, so that rows start on bank pairs 0, 12, 24 = 8, 36 = 4 and the 16 cells
+// of an x plane (a quarter wavefront) meet 16 pairs; field rows take 8 floats and planes end with 4
+// more, so that the 32 cells of two planes meet 32 banks.  Other shapes: rows as they are, planes
+// padded by 4.  128^3 x 16 ppc two-stream plasma, TSC Esirkepov kernel: 1.77 ms with padded planes
+// alone, 1.61 ms with these, 1.58 ms with esk_stay's shapes; QCAP keeps five workgroups on a CU.
+__host__ __device__ inline TileStrides tile_strides(bool c4, const int its[3], const int dts[3])
+{
+    TileStrides t;
+    t.isy = c4 ? 8 : its[2];
+    t.isx = c4 ? 6 * 8 * its[1] + 4 : its[1] * its[2] + 4;
+    t.itn = c4 ? 8 * its[1] : its[0] * t.isx;
+    t.ni = c4 ? its[0] * t.isx : 6 * t.itn;
+    t.dsy = c4 ? 28 : dts[2];
+    t.dsx = c4 ? 8 * 28 : dts[1] * dts[2] + 4;
+    t.dtn = c4 ? 8 : dts[0] * t.dsx;
+    t.nj = c4 ? dts[0] * t.dsx : 3 * t.dtn;
+    return t;
+}
 
 __device__ __forceinline__ bool colloc(int comp, int d)
 {
@@ -280,42 +302,78 @@ __device__ __forceinline__ void esirkepov_window(double* jt, int dtn, int dsx, i
     }
 }
 
-// Esirkepov deposit of two particles P and Q on one K x K x K window (neither changes its node):
-// every tile node receives the sum of both particles' terms with one atomic.  kqQ = 0 (and
-// finite Q shapes) deposits P alone.
-template <int K>
-__device__ __forceinline__ void esirkepov_pair(double* jt, int dtn, int sx, int sy, const int wb[3], const float S0P[3][4],
-                                               const float DSP[3][4], const float kqP[3], const float S0Q[3][4],
-                                               const float DSQ[3][4], const float kqQ[3])
+// A particle that keeps its node in every dimension: window base w, old shape S0 and shape change
+// DS on its K nodes a dimension: esk_shapes without a window of both shapes to place them in, so
+// without its selects.
+template <int SHAPE>
+__device__ __forceinline__ void esk_base(const int l[3], const float o[3], int w[3])
 {
+#pragma unroll
+    for (int d = 0; d < 3; d++) w[d] = SHAPE == PK_TSC || o[d] < 0.5f ? l[d] + 1 : l[d] + 2;
+}
+
+template <int SHAPE, int K>
+__device__ __forceinline__ void esk_stay_shapes(const float o[3], const float on[3], float S0[3][K], float DS[3][K])
+{
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const float s0 = o[d] - 0.5f, s1 = on[d] - 0.5f;
+        if (SHAPE == PK_TSC) {
+            float w0[3], w1[3];
+            tsc_w(s0, w0);
+            tsc_w(s1, w1);
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                asm("" : "+v"(w1[k]));      // rounded before the difference, as in esk_shapes
+                S0[d][k] = w0[k];
+                DS[d][k] = w1[k] - w0[k];
+            }
+        } else {
+            const float f0 = s0 < 0.0f ? s0 + 1.0f : s0, f1 = s1 < 0.0f ? s1 + 1.0f : s1;
+            S0[d][0] = 1.0f - f0;
+            S0[d][1] = f0;
+            DS[d][0] = (1.0f - f1) - (1.0f - f0);
+            DS[d][1] = f1 - f0;
+        }
+    }
+}
+
+// Esirkepov deposit of a staying particle P, or (PAIR) of two on one K x K x K window: every tile
+// node receives the sum of both particles' terms with one atomic.  qwQ = 0 (and finite offsets of Q)
+// deposits P alone.
+template <int SHAPE, bool PAIR>
+__device__ __forceinline__ void esk_stay(double* jt, int dtn, int sx, int sy, const int w[3], const float oP[3],
+                                         const float onP[3], float qwP, const float oQ[3], const float onQ[3], float qwQ,
+                                         const float hdt[3])
+{
+    constexpr int K = SHAPE == PK_TSC ? 3 : 2;
     const int st[3] = {sx, sy, 1};
-    const int orig = wb[0] * sx + wb[1] * sy + wb[2];
+    const int orig = w[0] * sx + w[1] * sy + w[2];
     const float third = 1.0f / 3.0f;
+    float S0P[3][K], DSP[3][K], S0Q[3][K] = {}, DSQ[3][K] = {};
+    esk_stay_shapes<SHAPE>(oP, onP, S0P, DSP);
+    if (PAIR) esk_stay_shapes<SHAPE>(oQ, onQ, S0Q, DSQ);
 #pragma unroll
     for (int comp = 0; comp < 3; comp++) {
         const int d1 = (comp + 1) % 3, d2 = (comp + 2) % 3;
-        float AP[K], BP[K], AQ[K], BQ[K];
-#pragma unroll
-        for (int p = 0; p < K; p++) {
-            AP[p] = kqP[comp] * (S0P[d1][p] + 0.5f * DSP[d1][p]);
-            BP[p] = kqP[comp] * (0.5f * S0P[d1][p] + third * DSP[d1][p]);
-            AQ[p] = kqQ[comp] * (S0Q[d1][p] + 0.5f * DSQ[d1][p]);
-            BQ[p] = kqQ[comp] * (0.5f * S0Q[d1][p] + third * DSQ[d1][p]);
-        }
+        const float kP = -qwP * hdt[comp], kQ = -qwQ * hdt[comp];
         double* t = jt + comp * dtn + orig + st[comp];
 #pragma unroll
-        for (int p = 0; p < K; p++)
+        for (int p = 0; p < K; p++) {
+            const float AP = kP * (S0P[d1][p] + 0.5f * DSP[d1][p]), BP = kP * (0.5f * S0P[d1][p] + third * DSP[d1][p]);
+            const float AQ = kQ * (S0Q[d1][p] + 0.5f * DSQ[d1][p]), BQ = kQ * (0.5f * S0Q[d1][p] + third * DSQ[d1][p]);
 #pragma unroll
             for (int r = 0; r < K; r++) {
-                const float cp = AP[p] * S0P[d2][r] + BP[p] * DSP[d2][r];
-                const float cq = AQ[p] * S0Q[d2][r] + BQ[p] * DSQ[d2][r];
+                const float cp = AP * S0P[d2][r] + BP * DSP[d2][r];
+                const float cq = AQ * S0Q[d2][r] + BQ * DSQ[d2][r];
                 float cum = 0.0f;
 #pragma unroll
                 for (int a = 0; a < K - 1; a++) {
-                    cum += DSP[comp][a] * cp + DSQ[comp][a] * cq;
+                    cum += PAIR ? DSP[comp][a] * cp + DSQ[comp][a] * cq : DSP[comp][a] * cp;
                     atomicAdd(&t[a * st[comp] + p * st[d1] + r * st[d2]], (double)cum);
                 }
             }
+        }
     }
 }
 
@@ -384,15 +442,14 @@ __device__ __forceinline__ void particles_split_sc(const SplitArgs& A, long s)
         dts[d] = nn[d] + (PICA_CIC ? 3 : 4);
         dbase[d] = PICA_CIC ? m0[d] + 1 : m0[d];
     }
-    const int isx = its[1] * its[2] + IPAD, isy = its[2];
-    const int dsx = dts[1] * dts[2] + JPAD, dsy = dts[2];
-    const int itn = its[0] * isx;
-    const int dtn = dts[0] * dsx;
+    const TileStrides ts = tile_strides(NC == 4, its, dts);
+    const int isx = ts.isx, isy = ts.isy, itn = ts.itn;
+    const int dsx = ts.dsx, dsy = ts.dsy, dtn = ts.dtn;
     // every LDS pointer is smem + a byte offset, so that the compiler keeps DS instructions
     float* itile = (float*)smem;
-    const int joff = (int)((sizeof(float) * 6 * itn + 7) & ~(size_t)7);
+    const int joff = (int)((sizeof(float) * ts.ni + 7) & ~(size_t)7);
     double* jtile = (double*)(smem + joff);
-    uint64_t* mask = (uint64_t*)(smem + joff + sizeof(double) * 3 * dtn);   // mover bit per particle
+    uint64_t* mask = (uint64_t*)(smem + joff + sizeof(double) * ts.nj);   // mover bit per particle
     int* dircnt = (int*)(mask + sp.mask_words);                                 // 27 direction counts
     int* bad = dircnt + 27;
     int* qlen = dircnt + 28;                                                    // change-queue length
@@ -447,7 +504,7 @@ __device__ __forceinline__ void particles_split_sc(const SplitArgs& A, long s)
             }
         }
     }
-    for (int t = tid; t < 3 * dtn; t += BS) jtile[t] = 0.0;
+    for (int t = tid; t < ts.nj; t += BS) jtile[t] = 0.0;
     for (int t = tid; t < 27; t += BS) dircnt[t] = 0;
     if (tid == 0) {
         bad[0] = 0;
@@ -629,39 +686,31 @@ __device__ __forceinline__ void particles_split_sc(const SplitArgs& A, long s)
             if (c0 + 64 < n) mask[(c0 >> 6) + 1] = spread_bits((uint32_t)(ma >> 32)) | (spread_bits((uint32_t)(mbm >> 32)) << 1);
         }
         if (DEP == PK_ESIRKEPOV) {
-            constexpr int KS = SHAPE == PK_TSC ? 3 : 2;    // window without a node change
             overflow(A);
             overflow(B);
             const bool sa = A.ok && A.cls == 0, sb = B.ok && B.cls == 0;
-            const bool small[3] = {false, false, false};
-            float S0a[3][4] = {}, DSa[3][4] = {}, S0b[3][4] = {}, DSb[3][4] = {};
-            int wa[3] = {0, 0, 0}, wbb[3] = {0, 0, 0};
-            if (sa) esk_shapes<SHAPE>(A.l, A.sh, A.o, A.on, small, wa, S0a, DSa);
-            if (sb) esk_shapes<SHAPE>(B.l, B.sh, B.o, B.on, small, wbb, S0b, DSb);
-            const bool merge = sa && sb && wa[0] == wbb[0] && wa[1] == wbb[1] && wa[2] == wbb[2];
+            int wa[3], wb[3];
+            esk_base<SHAPE>(A.l, A.o, wa);
+            esk_base<SHAPE>(B.l, B.o, wb);
+            const bool merge = sa && sb && wa[0] == wb[0] && wa[1] == wb[1] && wa[2] == wb[2];
             if (sa || sb) {
-                // A (with B when they share the window), or B alone when A has no small window
+                // A (with B when they share the window), or B alone when A has no small window; a B
+                // that takes no part counts with weight 0 and must be finite (a refused one may not be)
                 int wp[3];
-                float S0p[3][4], DSp[3][4], kp[3], kqq[3];
+                float op[3], onp[3], ob[3], onb[3];
 #pragma unroll
                 for (int d = 0; d < 3; d++) {
-                    wp[d] = sa ? wa[d] : wbb[d];
-#pragma unroll
-                    for (int k = 0; k < 4; k++) {
-                        S0p[d][k] = sa ? S0a[d][k] : S0b[d][k];
-                        DSp[d][k] = sa ? DSa[d][k] : DSb[d][k];
-                    }
-                    kp[d] = -(sa ? A.qw : B.qw) * sp.hdt[d];
-                    kqq[d] = merge ? -B.qw * sp.hdt[d] : 0.0f;
+                    wp[d] = sa ? wa[d] : wb[d];
+                    op[d] = sa ? A.o[d] : B.o[d];
+                    onp[d] = sa ? A.on[d] : B.on[d];
+                    ob[d] = sb ? B.o[d] : 0.0f;
+                    onb[d] = sb ? B.on[d] : 0.0f;
                 }
-                esirkepov_pair<KS>(jtile, dtn, dsx, dsy, wp, S0p, DSp, kp, S0b, DSb, kqq);
+                esk_stay<SHAPE, true>(jtile, dtn, dsx, dsy, wp, op, onp, sa ? A.qw : B.qw, ob, onb, merge ? B.qw : 0.0f, sp.hdt);
             }
             const bool second = sa && sb && !merge;
             if (__ballot(second)) {
-                if (second) {
-                    const float kb[3] = {-B.qw * sp.hdt[0], -B.qw * sp.hdt[1], -B.qw * sp.hdt[2]};
-                    esirkepov<KS, KS, KS>(jtile, dtn, dsx, dsy, wbb, S0b, DSb, kb);
-                }
+                if (second) esk_stay<SHAPE, false>(jtile, dtn, dsx, dsy, wb, B.o, B.on, B.qw, B.o, B.on, 0.0f, sp.hdt);
             }
         }
     }
@@ -696,14 +745,7 @@ __device__ __forceinline__ void particles_split_sc(const SplitArgs& A, long s)
     }
     // ---- movers: prefix over the mask words, copy to the outbox in index order, fill the holes
     const int words = (n + 63) >> 6;
-    if (tid == 0) {
-        long acc = 0;
-        for (int wd = 0; wd < words; wd++) {
-            wpre[wd] = acc;
-            acc += __popcll(mask[wd]);
-        }
-        wpre[words] = acc;
-    }
+    if (uwave == 0) pk_mask_prefix(mask, wpre, words, lane);
     __syncthreads();
     const int nmv = (int)wpre[words];
     const int nfinal = n - nmv;
@@ -1256,9 +1298,10 @@ size_t split_lds(const pk_ens* e, int shape, int dep, int mask_words)
         its[d] = e->ncps[d] + (shape == PK_TSC ? 3 : 2);
         dts[d] = e->ncps[d] + ((shape == PK_CIC && dep == PK_DIRECT) ? 3 : 4);
     }
-    const size_t joff = (sizeof(float) * 6 * its[0] * (its[1] * its[2] + IPAD) + 7) & ~(size_t)7;
-    const size_t base = joff + sizeof(double) * 3 * dts[0] * (dts[1] * dts[2] + JPAD) + sizeof(uint64_t) * mask_words +
-                        sizeof(int) * 32 + sizeof(long) * (mask_words + 1);
+    const TileStrides t = tile_strides(e->ncps[0] == 4 && e->ncps[1] == 4 && e->ncps[2] == 4, its, dts);
+    const size_t joff = (sizeof(float) * t.ni + 7) & ~(size_t)7;
+    const size_t base = joff + sizeof(double) * t.nj + sizeof(uint64_t) * mask_words + sizeof(int) * 32 +
+                        sizeof(long) * (mask_words + 1);
     if (dep != PK_ESIRKEPOV) return base + 16;
     return ((base + 15) & ~(size_t)15) + sizeof(int) * REC_WORDS * QCAP + 16;
 }
