@@ -29,7 +29,6 @@ __global__ void k_batch_clear(int* halt)
     if (threadIdx.x < PK_HALT_N) halt[threadIdx.x] = 0;
 }
 
-constexpr unsigned MASK_J = (1u << PK_JX) | (1u << PK_JY) | (1u << PK_JZ);
 
 // (ensemble, supercell) items: ensemble by ensemble in the XCD-aware supercell order of the
 // single-ensemble kernels, or all items by decreasing particle count (largest first); and the
@@ -75,16 +74,15 @@ int build_items(pk_batch* b, int shape)
 int enqueue_step(pk_batch* b)
 {
     int r;
-    if ((r = pk_batch_fields_launch(b, PK_BOP_ZERO_J, 0, 0))) return r;
+    if ((r = pk_batch_fields_launch(b, PK_BOP_ZERO_J))) return r;
     r = b->prec == PK_F64 ? pk_batch_f64_launch(b, b->dep) : pk_batch_split_launch(b, b->dep);
     if (r) return r;
-    // the periodic step's field forms: J fold gathered per cell, then its fill; Yee updates that
+    // the periodic step's field forms: J fold and fill per cell; Yee updates that
     // write their own ghost images (pk_step's sequence, bit for bit)
-    if ((r = pk_batch_fields_launch(b, PK_BOP_FOLD_J_P, 0, 0))) return r;
-    if ((r = pk_batch_fields_launch(b, PK_BOP_FILL, MASK_J, 0))) return r;
-    if ((r = pk_batch_fields_launch(b, PK_BOP_YEE_B_P, 0, 0))) return r;
-    if ((r = pk_batch_fields_launch(b, PK_BOP_YEE_E_P, 0, 0))) return r;
-    if ((r = pk_batch_fields_launch(b, PK_BOP_YEE_B_P, 0, 0))) return r;
+    if ((r = pk_batch_fields_launch(b, PK_BOP_FOLD_J_P))) return r;
+    if ((r = pk_batch_fields_launch(b, PK_BOP_YEE_B_P))) return r;
+    if ((r = pk_batch_fields_launch(b, PK_BOP_YEE_E_P))) return r;
+    if ((r = pk_batch_fields_launch(b, PK_BOP_YEE_B_P))) return r;
     if ((r = pk_batch_insert_launch(b))) return r;
     hipLaunchKernelGGL(k_batch_step_done, dim3(1), dim3(64), 0, b->ctx->stream, b->halt);
     PK_HIP(b->ctx, hipGetLastError());
@@ -211,12 +209,12 @@ int run(pk_batch* b, double dt, int shape, int dep, int nsteps)
         if ((r = set_base(done))) return r;
     }
     for (int j = 0; j < b->n(); j++) b->ens[j]->resorts = r0[j] + nsteps;
-    for (pk_ens* e : b->ens) {
-        int32_t fl[PK_NFLAGS];
-        if ((r = pk_flags_read(e, fl))) return r;
-        if (fl[PK_FLAG_ERR]) state_err = true;
-        if ((r = pk_flags_clear(e))) return r;
-    }
+    // one wait for all of them: a copy and a wait each took 1 ms for 64 plasmas
+    for (int j = 0; j < b->n(); j++)
+        if ((r = pk_flags_take(b->ens[j], b->flags_host + (size_t)j * PK_NFLAGS))) return r;
+    PK_HIP(c, hipStreamSynchronize(c->stream));
+    for (int j = 0; j < b->n(); j++)
+        if (b->flags_host[(size_t)j * PK_NFLAGS + PK_FLAG_ERR]) state_err = true;
     if (state_err)
         return pk_fail(c, PK_E_STATE,
                        "batch step: a particle was not finite or moved further than its tile allows "
@@ -359,8 +357,10 @@ int pk_batch_create(pk_ctx* c, int n, pk_ens* const* ens, pk_grid* const* grids,
     b->grids.assign(grids, grids + n);
     b->shapes.assign(n, -1);
     for (int d = 0; d < 3; d++) b->ncps0[d] = ens[0]->ncps[d];
-    if (hipMalloc((void**)&b->halt, sizeof(int) * PK_HALT_N) != hipSuccess) {
+    if (hipMalloc((void**)&b->halt, sizeof(int) * PK_HALT_N) != hipSuccess ||
+        hipHostMalloc((void**)&b->flags_host, sizeof(int32_t) * PK_NFLAGS * n, hipHostMallocDefault) != hipSuccess) {
         (void)hipGetLastError();
+        if (b->halt) (void)hipFree(b->halt);
         delete b;
         return pk_fail(c, PK_E_ALLOC, "pk_batch_create: hipMalloc failed");
     }
@@ -376,6 +376,7 @@ void pk_batch_destroy(pk_batch* b)
     for (void* p : {(void*)b->items, (void*)b->citems[0], (void*)b->citems[1], b->pjobs, b->ijobs, b->fjobs,
                     (void*)b->fstart, (void*)b->halt, b->iljobs, (void*)b->ilbase})
         if (p) (void)hipFree(p);
+    if (b->flags_host) (void)hipHostFree(b->flags_host);
     delete b;
 }
 

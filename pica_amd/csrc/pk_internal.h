@@ -250,12 +250,12 @@ __device__ __forceinline__ long pk_xcd_supercell(long b, int chunk)
 // ---- many ensembles stepped together (pk_batch_*) ----
 // Work of one stage for every ensemble goes into one launch: the particle and insert kernels
 // walk a list of (ensemble, supercell) items, the field kernels a per-ensemble block prefix.
-// work ranges of the batched field kernels: all cells, ghost cells, physical cells, physical cells
-// within the ghost width of a face
-enum { PK_BSTAGE_CELLS = 0, PK_BSTAGE_FILL = 1, PK_BSTAGE_PHYS = 2, PK_BSTAGE_FACE = 3, PK_BSTAGES = 4 };
-// the periodic step's field operations: J zero, ghost fill, Yee updates that write their own ghost
-// images, the J fold gathered per cell
-enum { PK_BOP_ZERO_J = 0, PK_BOP_FILL, PK_BOP_YEE_E_P, PK_BOP_YEE_B_P, PK_BOP_FOLD_J_P };
+// work ranges of the batched field kernels: all cells, physical cells, physical cells within the ghost
+// width of a face
+enum { PK_BSTAGE_CELLS = 0, PK_BSTAGE_PHYS = 1, PK_BSTAGE_FACE = 2, PK_BSTAGES = 3 };
+// the periodic step's field operations: J zero, Yee updates that write their own ghost images, the J
+// fold gathered per cell with the fill of its ghosts
+enum { PK_BOP_ZERO_J = 0, PK_BOP_YEE_E_P, PK_BOP_YEE_B_P, PK_BOP_FOLD_J_P };
 // device halt words of a batch: every batched kernel returns at once while STOP is set; an insert
 // overflow sets PENDING, which the step's last kernel turns into STOP (else it counts the step in DONE)
 enum { PK_HALT_STOP = 0, PK_HALT_DONE = 1, PK_HALT_PENDING = 2, PK_HALT_N = 4 };
@@ -289,13 +289,14 @@ struct pk_batch {
     int64_t* ilbase = nullptr; // per ensemble: re-sort count at the start of the current pass
     std::vector<int64_t> ilbase_host;
     int ilperiod = 0;          // interleave period captured by the prepared step (0: none)
+    int32_t* flags_host = nullptr;     // pinned: every ensemble's flags after a run
     hipGraphExec_t exec = nullptr;
     int n() const { return (int)ens.size(); }
 };
 // replace a device buffer by a copy of host data (outside any capture)
 int pk_batch_upload(pk_batch* b, void** dst, const void* src, size_t bytes);
 int pk_batch_fields_prepare(pk_batch* b, double dt);
-int pk_batch_fields_launch(pk_batch* b, int op, unsigned mask, int d);
+int pk_batch_fields_launch(pk_batch* b, int op);
 int pk_batch_shape_of(const pk_batch* b, int i, int shape);   // form factor of ensemble i in a run
 int pk_batch_split_prepare(pk_batch* b, double dt, int shape, int dep);
 int pk_batch_split_launch(pk_batch* b, int dep);
@@ -317,6 +318,8 @@ int pk_ens_resort_begin(pk_ens* e);
 int pk_ens_interleave_f64_launch(pk_ens* e);
 int pk_ens_resort_end(pk_ens* e);
 int pk_flags_clear(pk_ens* e);
+// queues one launch that moves the ensemble's flags to pinned host memory and clears them on the device
+int pk_flags_take(pk_ens* e, int32_t* pinned);
 int pk_ens_usable(pk_ens* e);               // PK_E_STATE after a failed re-sort rebuild
 int pk_ens_rebuild_after_overflow(pk_ens* e);   // rebuild of an overflowed re-sort; marks failure
 
@@ -333,8 +336,8 @@ int pk_field_ghost(pk_grid* g, int ops);
 // fill of that field's ghosts, in one launch over the physical cells
 #define PK_MAX_PERIODIC_GHOST 2
 int pk_field_yee_periodic(pk_grid* g, double dt, bool e_update);
-// the periodic step's J fold (physical cells bit-identical to PK_FOLD_J, in one launch; the ghosts
-// then hold stale values), followed by PK_FILL_J when fill
+// the periodic step's J fold (physical cells bit-identical to PK_FOLD_J), with PK_FILL_J in the same
+// launch when fill; without it the ghosts hold stale values
 int pk_field_fold_fill_j(pk_grid* g, bool fill);
 int pk_particles_launch(pk_ens* e, pk_grid* g, double dt, int shape, int dep);
 int pk_ens_insert_launch(pk_ens* e);
