@@ -197,6 +197,16 @@ struct EnsGeom {
 };
 
 // 3D cell of a linear physical cell index 0 <= c < 2^31 (z fastest)
+// Tile strides of supercells of one cell in z (two-dimensional runs).  Their rows are 3 to 5 nodes long, and
+// natural strides put a wavefront's neighbouring cells (y fastest, then x) on every fourth LDS bank.  An odd
+// row stride, and a plane stride that continues the progression over the `cells` rows that hold cells,
+// give any `banks` (a power of two) consecutive cells distinct ones.
+__host__ __device__ inline int pk_flat_row(int nodes) { return nodes | 1; }
+__host__ __device__ inline int pk_flat_plane(int rows, int row, int cells, int banks)
+{
+    return rows * row + (((cells - rows) * row) & (banks - 1));
+}
+
 // position of the k-th (from 0) set bit of m, k < popcount(m): popcount halving, 6 steps
 __device__ __forceinline__ int pk_select_bit(uint64_t m, int k)
 {

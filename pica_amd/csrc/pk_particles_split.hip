@@ -43,18 +43,18 @@ struct TileStrides {
 // so), and both tiles lay them on distinct LDS banks: the three components of a J row lie side by
 // side, 28 doubles a row, so that rows start on bank pairs 0, 12, 24 = 8, 36 = 4 and the 16 cells
 // of an x plane (a quarter wavefront) meet 16 pairs; field rows take 8 floats and planes end with 4
-// more, so that the 32 cells of two planes meet 32 banks.  Other shapes: rows as they are, planes
-// padded by 4.  128^3 x 16 ppc two-stream plasma, TSC Esirkepov kernel: 1.77 ms with padded planes
+// more, so that the 32 cells of two planes meet 32 banks.  Supercells of one cell in z with `flat` cells
+// in y (0: not those): pk_flat_row's strides.  Other shapes: rows as they are, planes padded by 4.  128^3 x 16 ppc two-stream plasma, TSC Esirkepov kernel: 1.77 ms with padded planes
 // alone, 1.61 ms with these, 1.58 ms with esk_stay's shapes; QCAP keeps five workgroups on a CU.
-__host__ __device__ inline TileStrides tile_strides(bool c4, const int its[3], const int dts[3])
+__host__ __device__ inline TileStrides tile_strides(bool c4, int flat, const int its[3], const int dts[3])
 {
     TileStrides t;
-    t.isy = c4 ? 8 : its[2];
-    t.isx = c4 ? 6 * 8 * its[1] + 4 : its[1] * its[2] + 4;
+    t.isy = c4 ? 8 : flat ? pk_flat_row(its[2]) : its[2];
+    t.isx = c4 ? 6 * 8 * its[1] + 4 : flat ? pk_flat_plane(its[1], t.isy, flat, 32) : its[1] * its[2] + 4;
     t.itn = c4 ? 8 * its[1] : its[0] * t.isx;
     t.ni = c4 ? its[0] * t.isx : 6 * t.itn;
-    t.dsy = c4 ? 28 : dts[2];
-    t.dsx = c4 ? 8 * 28 : dts[1] * dts[2] + 4;
+    t.dsy = c4 ? 28 : flat ? pk_flat_row(dts[2]) : dts[2];
+    t.dsx = c4 ? 8 * 28 : flat ? pk_flat_plane(dts[1], t.dsy, flat, 16) : dts[1] * dts[2] + 4;
     t.dtn = c4 ? 8 : dts[0] * t.dsx;
     t.nj = c4 ? dts[0] * t.dsx : 3 * t.dtn;
     return t;
@@ -442,7 +442,7 @@ __device__ __forceinline__ void particles_split_sc(const SplitArgs& A, long s)
         dts[d] = nn[d] + (PICA_CIC ? 3 : 4);
         dbase[d] = PICA_CIC ? m0[d] + 1 : m0[d];
     }
-    const TileStrides ts = tile_strides(NC == 4, its, dts);
+    const TileStrides ts = tile_strides(NC == 4, NC == 0 && eg.ncps[2] == 1 ? eg.ncps[1] : 0, its, dts);
     const int isx = ts.isx, isy = ts.isy, itn = ts.itn;
     const int dsx = ts.dsx, dsy = ts.dsy, dtn = ts.dtn;
     // every LDS pointer is smem + a byte offset, so that the compiler keeps DS instructions
@@ -1298,7 +1298,7 @@ size_t split_lds(const pk_ens* e, int shape, int dep, int mask_words)
         its[d] = e->ncps[d] + (shape == PK_TSC ? 3 : 2);
         dts[d] = e->ncps[d] + ((shape == PK_CIC && dep == PK_DIRECT) ? 3 : 4);
     }
-    const TileStrides t = tile_strides(e->ncps[0] == 4 && e->ncps[1] == 4 && e->ncps[2] == 4, its, dts);
+    const TileStrides t = tile_strides(e->ncps[0] == 4 && e->ncps[1] == 4 && e->ncps[2] == 4, e->ncps[2] == 1 ? e->ncps[1] : 0, its, dts);
     const size_t joff = (sizeof(float) * t.ni + 7) & ~(size_t)7;
     const size_t base = joff + sizeof(double) * t.nj + sizeof(uint64_t) * mask_words + sizeof(int) * 32 +
                         sizeof(long) * (mask_words + 1);
