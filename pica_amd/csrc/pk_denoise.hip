@@ -418,31 +418,39 @@ __global__ void __launch_bounds__(256) k_wgrad(Vol V, const uint16_t* __restrict
     }
 }
 
-// dW[t][ci][co] and db[co] += sum over the nwg workgroups' tiles; blockIdx.y takes every
-// gridDim.y-th group of 4 workgroups, so a weight receives gridDim.y atomic adds
+// dW[t][ci][co] and db[co] += sum over the nwg workgroups' tiles, in one order whatever the launch: WS_PARTS
+// strided sums, those by fours, and the fours with the gradient in FP64.  So the same inputs give the same bits, as
+// training needs: a last bit that moves flips a BF16 weight sooner or later, and two runs then part (with the fours
+// added by FP32 atomics in any order, by up to 5e-6 of the parameters after 32 iterations on 8 crops of 32^3 and 4e-5
+// after 96).  Reading the tiles bounds it (512 of them, 14.7 MB with CIN = 16), so a thread has eight loads under way:
+// 4.4 us (CIN = 4: 3.9 us), against 7.2 us one by one and 6.8 us with the atomics.
+constexpr int WS_PARTS = 32, WS_ELEMS = 32;
+
 template <int CIN>
-__global__ void __launch_bounds__(256) k_wgrad_sum(int nwg, const float* __restrict__ part, int cin, int cout,
-                                                   float* __restrict__ dW, float* __restrict__ db)
+__global__ void __launch_bounds__(WS_PARTS* WS_ELEMS) k_wgrad_sum(int nwg, const float* __restrict__ part, int cin,
+                                                                  int cout, float* __restrict__ dW,
+                                                                  float* __restrict__ db)
 {
     constexpr int NT = CIN == 16 ? WG_TILES16 : WG_TILES4, NE = (NT + 1) * 256;
-    const int lane = threadIdx.x & 63, p = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
+    static_assert(NE % WS_ELEMS == 0, "whole workgroups");
+    const int e = threadIdx.x % WS_ELEMS, p = threadIdx.x / WS_ELEMS;
+    const int i = blockIdx.x * WS_ELEMS + e;
     float s = 0.0f;
-    if (i < NE)
-        for (int w = 4 * blockIdx.y + p; w < nwg; w += 4 * gridDim.y) s += part[(long)w * NE + i];
-    __shared__ float red[4][64];
-    red[p][lane] = s;
+#pragma unroll 8
+    for (int w = p; w < nwg; w += WS_PARTS) s += part[(long)w * NE + i];
+    __shared__ float red[WS_PARTS][WS_ELEMS];
+    red[p][e] = s;
     __syncthreads();
-    if (p != 0 || i >= NE) return;
-    s = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+    if (p != 0) return;
     const int tile = i / 256, row = (i / 16) % 16, co = i % 16;
-    if (s == 0.0f || co >= cout) return;
-    if (tile == NT) {
-        if (row == 0) atomicAdd(&db[co], s);
-        return;
-    }
+    if (co >= cout || (tile == NT && row != 0)) return;
     const int tap = CIN == 16 ? tile : 4 * tile + row / 4, ci = CIN == 16 ? row : row % 4;
-    if (tap < 27 && ci < cin) atomicAdd(&dW[((long)tap * cin + ci) * cout + co], s);
+    if (tile != NT && (tap >= 27 || ci >= cin)) return;
+    float* const at = tile == NT ? db + co : dW + ((long)tap * cin + ci) * cout + co;
+    double sum = *at;
+#pragma unroll
+    for (int k = 0; k < WS_PARTS; k += 4) sum += red[k][e] + red[k + 1][e] + red[k + 2][e] + red[k + 3][e];
+    *at = (float)sum;
 }
 
 // weights -> MFMA B fragments of v_mfma_f32_16x16x32_bf16, wf[kc][lane][8].  Effective layer:
@@ -721,12 +729,12 @@ int wgrad(pk_dn* d, const Vol& V, const uint16_t* in, int cin_pad, int cin, cons
     const int nwg = (int)(total < WGRAD_WG_MAX ? total : WGRAD_WG_MAX);
     if (cin_pad == 16) {
         hipLaunchKernelGGL(k_wgrad<16>, dim3(nwg), dim3(256), wgrad_lds(16), s, V, in, g, gpad, cout, d->part);
-        hipLaunchKernelGGL(k_wgrad_sum<16>, dim3((WG_TILES16 + 1) * 256 / 64, 8), dim3(256), 0, s, nwg, d->part, cin,
-                           cout, dW, db);
+        hipLaunchKernelGGL(k_wgrad_sum<16>, dim3((WG_TILES16 + 1) * 256 / WS_ELEMS), dim3(WS_PARTS * WS_ELEMS), 0, s,
+                           nwg, d->part, cin, cout, dW, db);
     } else {
         hipLaunchKernelGGL(k_wgrad<4>, dim3(nwg), dim3(256), wgrad_lds(4), s, V, in, g, gpad, cout, d->part);
-        hipLaunchKernelGGL(k_wgrad_sum<4>, dim3((WG_TILES4 + 1) * 256 / 64, 8), dim3(256), 0, s, nwg, d->part, cin,
-                           cout, dW, db);
+        hipLaunchKernelGGL(k_wgrad_sum<4>, dim3((WG_TILES4 + 1) * 256 / WS_ELEMS), dim3(WS_PARTS * WS_ELEMS), 0, s,
+                           nwg, d->part, cin, cout, dW, db);
     }
     PK_HIP(d->ctx, hipGetLastError());
     return PK_OK;
