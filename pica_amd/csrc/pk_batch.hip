@@ -317,6 +317,15 @@ int pk_batch_shape_of(const pk_batch* b, int i, int shape)
     return shape == PK_SHAPE_PER_INSTANCE ? b->shapes[(size_t)i] : shape;
 }
 
+int pk_batch_cube(const pk_batch* b)
+{
+    const int edge = b->ens[0]->ncps[0];
+    for (const pk_ens* e : b->ens)
+        for (int d = 0; d < 3; d++)
+            if (e->ncps[d] != edge) return 0;
+    return edge;
+}
+
 int pk_batch_upload(pk_batch* b, void** dst, const void* src, size_t bytes)
 {
     if (*dst) (void)hipFree(*dst);

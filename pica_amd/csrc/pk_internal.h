@@ -308,6 +308,9 @@ int pk_batch_upload(pk_batch* b, void** dst, const void* src, size_t bytes);
 int pk_batch_fields_prepare(pk_batch* b, double dt);
 int pk_batch_fields_launch(pk_batch* b, int op);
 int pk_batch_shape_of(const pk_batch* b, int i, int shape);   // form factor of ensemble i in a run
+// edge of the cubic supercells that every ensemble of the batch has, 0 where they differ (an ensemble may
+// take others between two runs) or are no cubes: which particle kernel's launch takes all of them
+int pk_batch_cube(const pk_batch* b);
 int pk_batch_split_prepare(pk_batch* b, double dt, int shape, int dep);
 int pk_batch_split_launch(pk_batch* b, int dep);
 int pk_batch_f64_prepare(pk_batch* b, double dt, int shape, int dep);

@@ -543,8 +543,8 @@ StepParams step_params(const pk_ens* e, double dt)
 // 1.38 ms against 1.54 ms with strides read at run time)
 bool cube4(const pk_ens* e) { return e->ncps[0] == 4 && e->ncps[1] == 4 && e->ncps[2] == 4; }
 
-// dynamic LDS of k_particles: field and J tiles, mover mask, counters, mask prefix
-size_t f64_lds(const pk_ens* e, int shape, int dep, int mask_words)
+// dynamic LDS of k_particles (c4: its form for 4^3 supercells): field and J tiles, mover mask, counters, mask prefix
+size_t f64_lds(const pk_ens* e, bool c4, int shape, int dep, int mask_words)
 {
     const bool flat = e->ncps[2] == 1;
     int its[3], dts[3];
@@ -552,7 +552,6 @@ size_t f64_lds(const pk_ens* e, int shape, int dep, int mask_words)
         its[d] = e->ncps[d] + (shape == PK_CIC ? 2 : 3);
         dts[d] = e->ncps[d] + ((shape == PK_CIC && dep == PK_DIRECT) ? 3 : 4);
     }
-    const bool c4 = cube4(e);
     const size_t ip = flat ? pk_flat_plane(its[1], pk_flat_row(its[2]), e->ncps[1], 16) : its[1] * its[2];
     const size_t dp = flat ? pk_flat_plane(dts[1], pk_flat_row(dts[2]), e->ncps[1], 16) : dts[1] * dts[2];
     const size_t tiles = 6 * its[0] * (c4 ? (size_t)ISX4 : ip) + 3 * dts[0] * (c4 ? (size_t)DSX4 : dp);
@@ -582,7 +581,7 @@ int launch(pk_ens* e, pk_grid* g, double dt)
 {
     EnsGeom eg = ens_geom(e);
     const StepParams sp = step_params(e, dt);
-    const size_t lds = f64_lds(e, SHAPE, DEP, sp.mask_words);
+    const size_t lds = f64_lds(e, NC == 4, SHAPE, DEP, sp.mask_words);
     if (lds > 160 * 1024)
         return pk_fail(e->ctx, PK_E_CAPACITY, "particle step: supercell too large for LDS");
     const unsigned nblocks = (unsigned)(PK_XCD * (long)eg.xcd_chunk);
@@ -623,7 +622,7 @@ int launch_nc(pk_ens* e, pk_grid* g, double dt)
 template <int SHAPE, int DEP>
 int batch_go_nc(pk_batch* b, bool prepare)
 {
-    return cube4(b->ens[0]) ? batch_go<SHAPE, DEP, 4>(b, prepare) : batch_go<SHAPE, DEP, 0>(b, prepare);
+    return pk_batch_cube(b) == 4 ? batch_go<SHAPE, DEP, 4>(b, prepare) : batch_go<SHAPE, DEP, 0>(b, prepare);
 }
 
 // every form factor present, one launch each
@@ -656,13 +655,14 @@ int pk_batch_f64_prepare(pk_batch* b, double dt, int shape, int dep)
 {
     const int n = b->n();
     std::vector<F64Args> jobs(n);
+    const bool c4 = pk_batch_cube(b) == 4;
     b->cplds[0] = b->cplds[1] = 0;
     for (int i = 0; i < n; i++) {
         pk_ens* e = b->ens[i];
         const StepParams sp = step_params(e, dt);
         jobs[i] = f64_args(e, b->grids[i], ens_geom(e), sp);
         const int sh = pk_batch_shape_of(b, i, shape);
-        const size_t l = f64_lds(e, sh, dep, sp.mask_words);
+        const size_t l = f64_lds(e, c4, sh, dep, sp.mask_words);
         if (l > b->cplds[sh]) b->cplds[sh] = l;
     }
     if (b->cplds[0] > 160 * 1024 || b->cplds[1] > 160 * 1024)

@@ -1290,15 +1290,15 @@ __global__ void __launch_bounds__(PK_BLOCK) k_esk_sorted(GridView<float> g, EnsG
     }
 }
 
-// dynamic LDS of k_particles_split: field tile, FP64 J tile, mover mask, counters, mask prefix
-size_t split_lds(const pk_ens* e, int shape, int dep, int mask_words)
+// dynamic LDS of k_particles_split (c4: its form for 4^3 supercells): field tile, FP64 J tile, mover mask, counters, mask prefix
+size_t split_lds(const pk_ens* e, bool c4, int shape, int dep, int mask_words)
 {
     int its[3], dts[3];
     for (int d = 0; d < 3; d++) {
         its[d] = e->ncps[d] + (shape == PK_TSC ? 3 : 2);
         dts[d] = e->ncps[d] + ((shape == PK_CIC && dep == PK_DIRECT) ? 3 : 4);
     }
-    const TileStrides t = tile_strides(e->ncps[0] == 4 && e->ncps[1] == 4 && e->ncps[2] == 4, e->ncps[2] == 1 ? e->ncps[1] : 0, its, dts);
+    const TileStrides t = tile_strides(c4, e->ncps[2] == 1 ? e->ncps[1] : 0, its, dts);
     const size_t joff = (sizeof(float) * t.ni + 7) & ~(size_t)7;
     const size_t base = joff + sizeof(double) * t.nj + sizeof(uint64_t) * mask_words + sizeof(int) * 32 +
                         sizeof(long) * (mask_words + 1);
@@ -1346,7 +1346,7 @@ int launch(pk_ens* e, pk_grid* g, double dt)
     EnsGeom eg = ens_geom(e);
     SplitParams sp;
     if (int r = split_params(e, dt, sp)) return r;
-    const size_t lds = split_lds(e, SHAPE, DEP, sp.mask_words);
+    const size_t lds = split_lds(e, NC == 4, SHAPE, DEP, sp.mask_words);
     if (lds > 160 * 1024) return pk_fail(e->ctx, PK_E_CAPACITY, "particle step: supercell too large for LDS");
     const unsigned nblocks = (unsigned)(PK_XCD * (long)eg.xcd_chunk);
     pk_ktimer tm(e->ctx, "particles");
@@ -1457,12 +1457,12 @@ int batch_go(pk_batch* b, bool prepare)
 template <int SHAPE, int DEP>
 int batch_go_nc(pk_batch* b, bool prepare)
 {
-    const pk_ens* e = b->ens[0];
-    const bool cube = e->ncps[0] == e->ncps[1] && e->ncps[1] == e->ncps[2];
-    if (cube && e->ncps[0] == 4) return batch_go<SHAPE, DEP, 4>(b, prepare);
-    if (cube && e->ncps[0] == 2) return batch_go<SHAPE, DEP, 2>(b, prepare);
-    if (cube && e->ncps[0] == 8) return batch_go<SHAPE, DEP, 8>(b, prepare);
-    return batch_go<SHAPE, DEP, 0>(b, prepare);
+    switch (pk_batch_cube(b)) {
+    case 4: return batch_go<SHAPE, DEP, 4>(b, prepare);
+    case 2: return batch_go<SHAPE, DEP, 2>(b, prepare);
+    case 8: return batch_go<SHAPE, DEP, 8>(b, prepare);
+    default: return batch_go<SHAPE, DEP, 0>(b, prepare);
+    }
 }
 
 // every form factor present, one launch each
@@ -1495,6 +1495,7 @@ int pk_batch_split_prepare(pk_batch* b, double dt, int shape, int dep)
 {
     const int n = b->n();
     std::vector<SplitArgs> jobs(n);
+    const bool c4 = pk_batch_cube(b) == 4;
     b->cplds[0] = b->cplds[1] = 0;
     for (int i = 0; i < n; i++) {
         pk_ens* e = b->ens[i];
@@ -1502,7 +1503,7 @@ int pk_batch_split_prepare(pk_batch* b, double dt, int shape, int dep)
         if (int r = split_params(e, dt, sp)) return r;
         jobs[i] = split_args(e, b->grids[i], ens_geom(e), sp);
         const int sh = pk_batch_shape_of(b, i, shape);
-        const size_t l = split_lds(e, sh, dep, sp.mask_words);
+        const size_t l = split_lds(e, c4, sh, dep, sp.mask_words);
         if (l > b->cplds[sh]) b->cplds[sh] = l;
     }
     if (b->cplds[0] > 160 * 1024 || b->cplds[1] > 160 * 1024)
