@@ -251,6 +251,7 @@ int pk_species_set(pk_ctx* c, int ntypes, const double* mass, const double* char
     if (!c || ntypes <= 0 || !mass || !charge) return pk_fail(c, PK_E_ARG, "pk_species_set: bad arguments");
     c->mass.assign(mass, mass + ntypes);
     c->charge.assign(charge, charge + ntypes);
+    c->species++;
     return PK_OK;
 }
 

@@ -111,6 +111,9 @@ int prepare(pk_batch* b, double dt, int shape, int dep)
     b->dt = dt;
     b->shape = shape;
     b->dep = dep;
+    b->species = c->species;
+    b->layouts.clear();
+    for (const pk_ens* e : b->ens) b->layouts.push_back(e->layout);
     if (b->knob[PK_BATCH_GRAPH]) {
         const bool timing = c->timing;
         c->timing = false;      // no event records inside the capture
@@ -149,6 +152,15 @@ int check_args(pk_batch* b, double dt, int shape, int dep)
     return PK_OK;
 }
 
+// the prepared launches still hold what the ensembles and the species table are
+bool current(const pk_batch* b)
+{
+    if (b->dirty || b->species != b->ctx->species) return false;
+    for (int i = 0; i < b->n(); i++)
+        if (b->ens[i]->layout != b->layouts[i]) return false;
+    return true;
+}
+
 int run(pk_batch* b, double dt, int shape, int dep, int nsteps)
 {
     pk_ctx* c = b->ctx;
@@ -158,7 +170,7 @@ int run(pk_batch* b, double dt, int shape, int dep, int nsteps)
     const int period = b->ens[0]->posmode == PK_POS_SPLIT
                            ? (b->knob[PK_BATCH_INTERLEAVE] >= 0 ? b->knob[PK_BATCH_INTERLEAVE] : c->opt[PK_OPT_INTERLEAVE])
                            : 0;
-    if (b->dirty || dt != b->dt || shape != b->shape || dep != b->dep || period != b->ilperiod)
+    if (!current(b) || dt != b->dt || shape != b->shape || dep != b->dep || period != b->ilperiod)
         if ((r = prepare(b, dt, shape, dep))) return r;
     // re-sort counts before this run; each pass tells the interleave kernel where it starts
     std::vector<long> r0(b->n());
@@ -299,6 +311,7 @@ int snapshot_restore(pk_batch* b, const Snapshot& S)
         PK_HIP(c, hipMemcpyAsync(b->grids[i]->data, S.grids[i], grid_bytes(b->grids[i]), hipMemcpyDeviceToDevice,
                                  c->stream));
         e->maxcap = s.maxcap;
+        e->layout++;
         e->np = s.np;
         e->resorts = s.resorts;
         e->pending_movers = false;

@@ -704,6 +704,7 @@ int pk_ens_alloc(pk_ens* e, size_t capacity)
     e->outbox = o;
     e->odir = od;
     e->capacity = capacity;
+    e->layout++;
     return PK_OK;
 }
 
@@ -1265,6 +1266,7 @@ static int rebuild_from(pk_ens* e, long nent, DBuf& keys_in, DBuf& srcs_in, Fiel
     e->odir = nodir;
     e->capacity = (size_t)total_cap;
     e->maxcap = mc;
+    e->layout++;
     e->np = nent;
     e->pending_movers = false;
     e->failed = false;
@@ -1348,6 +1350,7 @@ int pk_ens_reshape(pk_ens* e, const int ncps[3])
         e->nsc[d] = nsc[d];
     }
     e->nsct = nsct;
+    e->layout++;
     return PK_OK;
 }
 
@@ -1504,6 +1507,7 @@ int pk_ens_load_impl(pk_ens* e, int ppc, double uth, double drift, double weight
     PK_HIP(c, hipGetLastError());
     if (nmodes > 0) PK_HIP(c, hipStreamSynchronize(c->stream));   // before the mode table is freed
     e->maxcap = (int)cap;
+    e->layout++;
     e->np = (int64_t)per_sc * e->nsct;
     e->pending_movers = false;
     e->failed = false;

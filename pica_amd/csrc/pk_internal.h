@@ -33,6 +33,7 @@ struct pk_ctx {
     hipStream_t stream = nullptr;
     std::string err;
     std::vector<double> mass, charge;   // ParticleTypes table
+    uint64_t species = 0;               // counts its changes
     bool timing = false;
     struct pending {
         std::string name;
@@ -96,6 +97,7 @@ struct pk_ens {
     int32_t* mvc = nullptr;      // nsct * 27 movers per direction class
     int32_t* flags = nullptr;    // PK_NFLAGS device flags
     int maxcap = 0;
+    uint64_t layout = 0;          // counts the changes of buffers, capacities and supercells
     int64_t np = 0;
     bool pending_movers = false;  // particle step done, re-sort not yet done
     bool resort_inflight = false; // insert and flag copy launched, flags not yet read
@@ -278,8 +280,11 @@ struct pk_batch {
     int knob[PK_BATCH_NKNOB] = {0, 1, 1, 0, -1, PK_BLOCK};
     int ncps0[3] = {0, 0, 0};  // supercell shape the ensembles had when the batch was created
     std::vector<int> shapes;   // per-ensemble form factor for PK_SHAPE_PER_INSTANCE (-1: unset)
-    // prepared launch state, valid while !dirty and (dt, shape, dep) are unchanged
+    // prepared launch state, valid while !dirty and (dt, shape, dep), the species table and the ensembles'
+    // layouts (each may be stepped, loaded or re-bucketed on its own between two runs) are unchanged
     bool dirty = true;
+    uint64_t species = 0;
+    std::vector<uint64_t> layouts;
     double dt = 0.0;
     int shape = -1, dep = -1;
     int2* items = nullptr;     // (ensemble, supercell) in launch order

@@ -221,6 +221,7 @@ int pk_ens_load(pk_ens* e, const char* path)
     PK_HIP(c, hipMemset(e->nmove, 0, sizeof(int32_t) * nsct));
     PK_HIP(c, hipMemset(e->flags, 0, sizeof(int32_t) * PK_NFLAGS));
     e->maxcap = maxcap;
+    e->layout++;
     e->np = np;
     e->pending_movers = false;
     e->failed = false;

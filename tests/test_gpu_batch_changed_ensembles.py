@@ -1,5 +1,6 @@
 """A batch whose ensembles changed between two runs, against stepping each pair on its own: supercells of one of them
-re-bucketed, so that the batch holds several shapes at once.
+re-bucketed, so that the batch holds several shapes at once; and, with nothing else that would prepare the launches
+again, particles uploaded, loaded from a snapshot, re-bucketed or stepped on their own, or other species.
 
 Same bounds as the batch tests: FP64 1e-12, FP32 2e-5 of the scale, supercell membership and particle order equal."""
 import numpy as np
@@ -39,3 +40,54 @@ def test_supercells_of_one_ensemble_change(ctx, prec, shape, dep, change):
         P.run(e, g, 0.5 * dt, 3, shape, dep)
     _same(prec, mine, ref, "re-bucketed")
     b.close()
+
+
+def _upload(ctx, pair, tmp_path, dt):
+    rng = np.random.default_rng(5)
+    e, _ = pair
+    n = 4000          # more than before: other buffers, other capacities
+    e.add(rng.random((n, 3)) * e.ncell, 0.05 * rng.standard_normal((n, 3)), 1e3 * (1.0 + np.arange(n) * 2.0 ** -20))
+
+
+def _reload(ctx, pair, tmp_path, dt):
+    pair[0].save(str(tmp_path / "e"))
+    pair[0].load(str(tmp_path / "e"))
+
+
+def _rebucket(ctx, pair, tmp_path, dt):
+    pair[0].set_supercells((2, 4, 2))
+
+
+def _own_steps(ctx, pair, tmp_path, dt):
+    pair[0].set_slack(0.0, 0)
+    pair[0].set_supercells((2, 2, 2))
+    P.run(pair[0], pair[1], dt, 3, P.TSC, P.ESIRKEPOV)         # overflows its supercells: rebuilt
+
+
+def _other_species(ctx, pair, tmp_path, dt):
+    ctx.set_species([3.0 * P.ELECTRON_MASS], [2.0 * P.ELECTRON_CHARGE])
+
+
+@pytest.mark.parametrize("prec", [P.F64, P.F32])
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("change", [_upload, _reload, _rebucket, _own_steps, _other_species])
+def test_changed_between_runs_of_one_dt(prec, graph, change, tmp_path):
+    _say("batch, %s between two runs, prec=%d graph=%d" % (change.__name__, prec, graph))
+    dt = courant_dt()
+    ctx = P.Context(0)
+    ctx.set_option(P.OPT_INTERLEAVE, 0)
+    if change is _other_species:
+        ctx.set_species([P.ELECTRON_MASS], [P.ELECTRON_CHARGE])
+    mine, ref = _pairs(ctx, prec), _pairs(ctx, prec)
+    b = P.Batch(ctx, mine)
+    b.set(P.BATCH_GRAPH, graph)
+    b.run(dt, 2, P.TSC, P.ESIRKEPOV)
+    for e, g in ref:
+        P.run(e, g, dt, 2, P.TSC, P.ESIRKEPOV)
+    for pair in (mine[1], ref[1]):
+        change(ctx, pair, tmp_path, dt)
+    b.run(dt, 3, P.TSC, P.ESIRKEPOV)
+    for e, g in ref:
+        P.run(e, g, dt, 3, P.TSC, P.ESIRKEPOV)
+    _same(prec, mine, ref, change.__name__)
+    ctx.close()
