@@ -336,11 +336,18 @@ __device__ __forceinline__ bool deposit_direct(const ScGeom& q, double* jt, cons
 // DS = d (m - 1/2), -2 m d, d (m + 1/2), currents through its two faces ~ d (1/2 - m), d (1/2 + m);
 // CIC: M = 1 - m, m, DS = -d, d, one face ~ d.
 // So a staying particle takes 54 (TSC) or 12 (CIC) LDS atomics on its own window.  One that changes node
-// waits in its lane's registers until four of the wavefront do (or its lane meets another), and is then
-// deposited by 16 lanes, one per transverse node pair, on the 4- or 3-node window of old and new shape.
+// takes the 4- or 3-node window of old and new shape.  Where few of a wavefront's 64 change, each waits in its
+// lane's registers until four do (or its lane meets another), and is then deposited by 16 lanes, one per
+// transverse node pair.  Four of them cost 44 LDS shuffles, so from ESK_MANY changers of the 64 on each is
+// deposited by its own lane at once.
 // 128^3 x 16 ppc two-stream plasma, whole kernel: TSC 3.82 -> 2.68 ms, CIC 2.06 -> 1.65 ms against adding every
 // particle's 4- (3-) node window, of which 3% of the particles need more than 3 (2) nodes a side; with the
 // changers in a workgroup queue instead of registers 2.84 ms (its pass after the push waits at a barrier).
+// Hot plasmas, 64^3 x 16 ppc, thermal u = 0.1, 0.3 and 2: TSC 444, 513, 593 us (16 lanes each always: 440, 580, 801;
+// every particle's window by its lane: 598, 638, 691), CIC 231, 248, 266 us (238, 330, 476; 282, 287, 303).
+// ESK_MANY 50% higher: TSC 447, 573, 596, CIC 239, 247, 270 us.
+template <int SHAPE>
+constexpr int ESK_MANY = SHAPE == PK_CIC ? 8 : 16;
 
 // lowest node of the shape at cell-centre coordinate xi, and the offset its closed form takes: from the
 // nearest node (TSC) or from the lower one (CIC)
@@ -420,6 +427,58 @@ __device__ __forceinline__ int esk_stay(const ScGeom& q, double* jt, const doubl
         }
     }
     return 0;
+}
+
+// deposits a particle on the window of its old and new shape (a node changer)
+template <int SHAPE>
+__device__ __forceinline__ void esk_window(const ScGeom& q, double* jt, const double x0[3], const double x1[3], double qw,
+                                           const double hdt[3])
+{
+    constexpr int KW = SHAPE == PK_CIC ? 3 : 4;
+    double M[3][KW], D[3][KW];
+    int w[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double off = q.nom[d] + 0.5;
+        double d0, d1, s0[3], s1[3];
+        const int a0 = esk_node<SHAPE>(x0[d] * q.inv[d] - off, d0), a1 = esk_node<SHAPE>(x1[d] * q.inv[d] - off, d1);
+        if (SHAPE == PK_CIC) {
+            s0[0] = 1.0 - d0; s0[1] = d0;
+            s1[0] = 1.0 - d1; s1[1] = d1;
+        } else {
+            tsc_w(d0, s0);
+            tsc_w(d1, s1);
+        }
+        w[d] = a0 < a1 ? a0 : a1;
+#pragma unroll
+        for (int k = 0; k < KW; k++) {
+            const double a = a0 > a1 ? (k ? s0[k - 1] : 0.0) : (k < KW - 1 ? s0[k] : 0.0);
+            const double b = a1 > a0 ? (k ? s1[k - 1] : 0.0) : (k < KW - 1 ? s1[k] : 0.0);
+            M[d][k] = 0.5 * (a + b);
+            D[d][k] = b - a;
+        }
+    }
+    const int st[3] = {q.dsx, q.dsy, 1};
+    double* t0 = jt + w[0] * q.dsx + w[1] * q.dsy + w[2];
+#pragma unroll
+    for (int comp = 0; comp < 3; comp++) {
+        const int d1 = (comp + 1) % 3, d2 = (comp + 2) % 3;
+        double cum[KW - 1];
+#pragma unroll
+        for (int a = 0; a < KW - 1; a++) cum[a] = -qw * hdt[comp] * D[comp][a] + (a ? cum[a - 1] : 0.0);
+        double* t = t0 + comp * q.dtn + st[comp];
+#pragma unroll
+        for (int p = 0; p < KW; p++) {
+            const double dp = (1.0 / 12.0) * D[d1][p];
+#pragma unroll
+            for (int r = 0; r < KW; r++) {
+                const double g = fma(M[d1][p], M[d2][r], dp * D[d2][r]);
+                if (g == 0.0) continue;      // a node pair that only a change in these dimensions reaches
+#pragma unroll
+                for (int a = 0; a < KW - 1; a++) atomicAdd(&t[a * st[comp] + p * st[d1] + r * st[d2]], cum[a] * g);
+            }
+        }
+    }
 }
 
 // a node changer by 16 lanes (every lane of the wavefront takes part; has = the lanes hold one): lane
