@@ -198,15 +198,43 @@ struct EnsGeom {
     FastDiv div12, div2;   // by ncell[1] * ncell[2] and by ncell[2]
 };
 
-// 3D cell of a linear physical cell index 0 <= c < 2^31 (z fastest)
 // Tile strides of supercells of one cell in z (two-dimensional runs).  Their rows are 3 to 5 nodes long, and
-// natural strides put a wavefront's neighbouring cells (y fastest, then x) on every fourth LDS bank.  An odd
-// row stride, and a plane stride that continues the progression over the `cells` rows that hold cells,
-// give any `banks` (a power of two) consecutive cells distinct ones.
-__host__ __device__ inline int pk_flat_row(int nodes) { return nodes | 1; }
-__host__ __device__ inline int pk_flat_plane(int rows, int row, int cells, int banks)
+// natural strides put a wavefront's neighbouring cells (y fastest, then x) on every fourth LDS bank where a row is
+// even.  Level 1: an odd row stride; level 2: and a plane stride that continues the progression over the `cells`
+// rows that hold cells, so that any `banks` (a power of two) consecutive cells have distinct ones; level 0: rows
+// as they are, planes padded by `pad`.
+__host__ __device__ inline int pk_flat_row(int level, int nodes) { return level ? nodes | 1 : nodes; }
+__host__ __device__ inline int pk_flat_plane(int level, int rows, int row, int cells, int banks, int pad)
 {
-    return rows * row + (((cells - rows) * row) & (banks - 1));
+    return rows * row + (level == 2 ? ((cells - rows) * row) & (banks - 1) : pad);
+}
+
+struct FlatLevels {
+    int field, j;
+};
+
+// The levels of a supercell's field and J tiles.  lds(levels): bytes of a workgroup; most: workgroups a CU that the
+// registers allow; even: the field tile's rows are even (TSC).  The highest levels that leave as many workgroups on a
+// CU as level 0 does, J first (its atomics cost more than reads), since a workgroup less costs more than the conflicts:
+// 504 x 504 x 16 ppc, us a step at level 0 / level 2 whatever the LDS / now: FP32 CIC Esirkepov 12 x 4 cells 207 / 226 /
+// 170, FP64 CIC direct 12 x 12 234 / 241 / 233, FP64 TSC direct 12 x 12 551 / 623 / 519.  Even rows of the field tile
+// (every fourth bank) cost more than one workgroup of three: FP64 TSC direct 9 x 9 545 us at level 0, 480 at level 2
+// with two workgroups.  6 x 6, where all levels fit: FP64 TSC direct 554 / 450 / 450, FP32 TSC Esirkepov 369 / 335 / 311.
+template <class F>
+inline FlatLevels pk_flat_levels(F lds, int most, bool even)
+{
+    constexpr size_t CU = 160 * 1024, GRAIN = 1280;      // LDS of a CU, and what it is given out in
+    auto fit = [&](FlatLevels f) {
+        const size_t n = CU / ((lds(f) + GRAIN - 1) / GRAIN * GRAIN);
+        return n < (size_t)most ? (int)n : most;
+    };
+    const int want = fit(FlatLevels{0, 0});
+    for (int lost = 0; lost <= (even && want >= 3 ? 1 : 0); lost++)
+        for (int k = 8; k > 0; k--)
+            if (k % 3 && fit(FlatLevels{k % 3, k / 3}) >= want - lost) return FlatLevels{k % 3, k / 3};
+    for (int j = 2; j > 0; j--)
+        if (fit(FlatLevels{0, j}) >= want) return FlatLevels{0, j};
+    return FlatLevels{0, 0};
 }
 
 // position of the k-th (from 0) set bit of m, k < popcount(m): popcount halving, 6 steps
@@ -243,6 +271,7 @@ __device__ __forceinline__ void pk_mask_prefix(const uint64_t* mask, long* pre, 
     if (lane == 0) pre[words] = run;
 }
 
+// 3D cell of a linear physical cell index 0 <= c < 2^31 (z fastest)
 __device__ __forceinline__ void cell_coords(int c, const EnsGeom& eg, int cc[3])
 {
     const int q12 = (int)fastdiv((uint32_t)c, eg.div12), q2 = (int)fastdiv((uint32_t)c, eg.div2);

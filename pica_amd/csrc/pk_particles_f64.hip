@@ -34,12 +34,10 @@ struct ScGeom {
     int isx, isy, itn, dsx, dsy, dtn;      // strides and size of one component's field and J tile
 };
 
-// NC == 4: 4^3 supercells (constant strides); NC == 0: any shape, natural strides or (flat) those of one cell
-// in z (252 x 180 x 24 ppc, 6 x 6 x 1 supercells, TSC direct: 163 -> 137 us)
+// NC == 4: 4^3 supercells (constant strides); NC == 0: any shape, with the strides of `flat`'s levels
 template <int SHAPE, int DEP, int NC>
-__device__ __forceinline__ void sc_geom(const GridView<double>& g, const EnsGeom& eg, const int sidx[3], ScGeom& q)
+__device__ __forceinline__ void sc_geom(const GridView<double>& g, const EnsGeom& eg, FlatLevels flat, const int sidx[3], ScGeom& q)
 {
-    const bool flat = NC == 0 && eg.ncps[2] == 1;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         const double step = g.step[d];
@@ -60,11 +58,11 @@ __device__ __forceinline__ void sc_geom(const GridView<double>& g, const EnsGeom
             q.dts[d] = n + 4;
         }
     }
-    q.isy = NC == 4 ? ISY4 : flat ? pk_flat_row(q.its[2]) : q.its[2];
-    q.isx = NC == 4 ? ISX4 : flat ? pk_flat_plane(q.its[1], q.isy, eg.ncps[1], 16) : q.its[1] * q.its[2];
+    q.isy = NC == 4 ? ISY4 : pk_flat_row(flat.field, q.its[2]);
+    q.isx = NC == 4 ? ISX4 : pk_flat_plane(flat.field, q.its[1], q.isy, eg.ncps[1], 16, 0);
     q.itn = q.its[0] * q.isx;
-    q.dsy = NC == 4 ? DSY4 : flat ? pk_flat_row(q.dts[2]) : q.dts[2];
-    q.dsx = NC == 4 ? DSX4 : flat ? pk_flat_plane(q.dts[1], q.dsy, eg.ncps[1], 16) : q.dts[1] * q.dts[2];
+    q.dsy = NC == 4 ? DSY4 : pk_flat_row(flat.j, q.dts[2]);
+    q.dsx = NC == 4 ? DSX4 : pk_flat_plane(flat.j, q.dts[1], q.dsy, eg.ncps[1], 16, 0);
     q.dtn = q.dts[0] * q.dsx;
 }
 
@@ -525,6 +523,7 @@ struct StepParams {
     double dt, coeff, q;
     double L[3], scinv[3], hdt[3];
     int mask_words;
+    FlatLevels flat;
 };
 
 // all arguments of one ensemble's particle step (one kernel argument, or one entry of a batch)
@@ -580,7 +579,9 @@ __global__ void __launch_bounds__(PK_BLOCK) k_particles_batch(const F64Args* __r
     }
 }
 
-StepParams step_params(const pk_ens* e, double dt)
+size_t f64_lds(const pk_ens* e, bool c4, int shape, int dep, int mask_words, FlatLevels flat);
+
+StepParams step_params(const pk_ens* e, double dt, int shape, int dep)
 {
     StepParams sp;
     sp.dt = dt;
@@ -594,6 +595,10 @@ StepParams step_params(const pk_ens* e, double dt)
         sp.hdt[d] = e->step[d] / dt;
     }
     sp.mask_words = (e->maxcap + PK_BLOCK + 63) / 64 + 1;
+    sp.flat = FlatLevels{0, 0};
+    if (e->ncps[2] == 1)
+        sp.flat = pk_flat_levels([&](FlatLevels f) { return f64_lds(e, false, shape, dep, sp.mask_words, f); },
+                                 shape == PK_CIC && dep == PK_DIRECT ? 4 : 3, shape == PK_TSC);
     return sp;
 }
 
@@ -603,16 +608,15 @@ StepParams step_params(const pk_ens* e, double dt)
 bool cube4(const pk_ens* e) { return e->ncps[0] == 4 && e->ncps[1] == 4 && e->ncps[2] == 4; }
 
 // dynamic LDS of k_particles (c4: its form for 4^3 supercells): field and J tiles, mover mask, counters, mask prefix
-size_t f64_lds(const pk_ens* e, bool c4, int shape, int dep, int mask_words)
+size_t f64_lds(const pk_ens* e, bool c4, int shape, int dep, int mask_words, FlatLevels flat)
 {
-    const bool flat = e->ncps[2] == 1;
     int its[3], dts[3];
     for (int d = 0; d < 3; d++) {
         its[d] = e->ncps[d] + (shape == PK_CIC ? 2 : 3);
         dts[d] = e->ncps[d] + ((shape == PK_CIC && dep == PK_DIRECT) ? 3 : 4);
     }
-    const size_t ip = flat ? pk_flat_plane(its[1], pk_flat_row(its[2]), e->ncps[1], 16) : its[1] * its[2];
-    const size_t dp = flat ? pk_flat_plane(dts[1], pk_flat_row(dts[2]), e->ncps[1], 16) : dts[1] * dts[2];
+    const size_t ip = pk_flat_plane(flat.field, its[1], pk_flat_row(flat.field, its[2]), e->ncps[1], 16, 0);
+    const size_t dp = pk_flat_plane(flat.j, dts[1], pk_flat_row(flat.j, dts[2]), e->ncps[1], 16, 0);
     const size_t tiles = 6 * its[0] * (c4 ? (size_t)ISX4 : ip) + 3 * dts[0] * (c4 ? (size_t)DSX4 : dp);
     return sizeof(double) * tiles + sizeof(uint64_t) * mask_words + sizeof(int) * 32 + sizeof(long) * (mask_words + 1) + 16;
 }
@@ -639,8 +643,8 @@ template <int SHAPE, int DEP, int NC>
 int launch(pk_ens* e, pk_grid* g, double dt)
 {
     EnsGeom eg = ens_geom(e);
-    const StepParams sp = step_params(e, dt);
-    const size_t lds = f64_lds(e, NC == 4, SHAPE, DEP, sp.mask_words);
+    const StepParams sp = step_params(e, dt, SHAPE, DEP);
+    const size_t lds = f64_lds(e, NC == 4, SHAPE, DEP, sp.mask_words, sp.flat);
     if (lds > 160 * 1024)
         return pk_fail(e->ctx, PK_E_CAPACITY, "particle step: supercell too large for LDS");
     const unsigned nblocks = (unsigned)(PK_XCD * (long)eg.xcd_chunk);
@@ -718,10 +722,10 @@ int pk_batch_f64_prepare(pk_batch* b, double dt, int shape, int dep)
     b->cplds[0] = b->cplds[1] = 0;
     for (int i = 0; i < n; i++) {
         pk_ens* e = b->ens[i];
-        const StepParams sp = step_params(e, dt);
-        jobs[i] = f64_args(e, b->grids[i], ens_geom(e), sp);
         const int sh = pk_batch_shape_of(b, i, shape);
-        const size_t l = f64_lds(e, c4, sh, dep, sp.mask_words);
+        const StepParams sp = step_params(e, dt, sh, dep);
+        jobs[i] = f64_args(e, b->grids[i], ens_geom(e), sp);
+        const size_t l = f64_lds(e, c4, sh, dep, sp.mask_words, sp.flat);
         if (l > b->cplds[sh]) b->cplds[sh] = l;
     }
     if (b->cplds[0] > 160 * 1024 || b->cplds[1] > 160 * 1024)

@@ -43,18 +43,19 @@ struct TileStrides {
 // so), and both tiles lay them on distinct LDS banks: the three components of a J row lie side by
 // side, 28 doubles a row, so that rows start on bank pairs 0, 12, 24 = 8, 36 = 4 and the 16 cells
 // of an x plane (a quarter wavefront) meet 16 pairs; field rows take 8 floats and planes end with 4
-// more, so that the 32 cells of two planes meet 32 banks.  Supercells of one cell in z with `flat` cells
-// in y (0: not those): pk_flat_row's strides.  Other shapes: rows as they are, planes padded by 4.  128^3 x 16 ppc two-stream plasma, TSC Esirkepov kernel: 1.77 ms with padded planes
-// alone, 1.61 ms with these, 1.58 ms with esk_stay's shapes; QCAP keeps five workgroups on a CU.
-__host__ __device__ inline TileStrides tile_strides(bool c4, int flat, const int its[3], const int dts[3])
+// more, so that the 32 cells of two planes meet 32 banks.  Other shapes: rows as they are and planes padded
+// by 4 (level 0), or for supercells of one cell in z the levels of `flat`, with `cells` cells in y.  128^3 x 16 ppc
+// two-stream plasma, TSC Esirkepov kernel: 1.77 ms with padded planes alone, 1.61 ms with these, 1.58 ms with
+// esk_stay's shapes; QCAP keeps five workgroups on a CU.
+__host__ __device__ inline TileStrides tile_strides(bool c4, FlatLevels flat, int cells, const int its[3], const int dts[3])
 {
     TileStrides t;
-    t.isy = c4 ? 8 : flat ? pk_flat_row(its[2]) : its[2];
-    t.isx = c4 ? 6 * 8 * its[1] + 4 : flat ? pk_flat_plane(its[1], t.isy, flat, 32) : its[1] * its[2] + 4;
+    t.isy = c4 ? 8 : pk_flat_row(flat.field, its[2]);
+    t.isx = c4 ? 6 * 8 * its[1] + 4 : pk_flat_plane(flat.field, its[1], t.isy, cells, 32, 4);
     t.itn = c4 ? 8 * its[1] : its[0] * t.isx;
     t.ni = c4 ? its[0] * t.isx : 6 * t.itn;
-    t.dsy = c4 ? 28 : flat ? pk_flat_row(dts[2]) : dts[2];
-    t.dsx = c4 ? 8 * 28 : flat ? pk_flat_plane(dts[1], t.dsy, flat, 16) : dts[1] * dts[2] + 4;
+    t.dsy = c4 ? 28 : pk_flat_row(flat.j, dts[2]);
+    t.dsx = c4 ? 8 * 28 : pk_flat_plane(flat.j, dts[1], t.dsy, cells, 16, 4);
     t.dtn = c4 ? 8 : dts[0] * t.dsx;
     t.nj = c4 ? dts[0] * t.dsx : 3 * t.dtn;
     return t;
@@ -396,6 +397,7 @@ struct SplitParams {
     float hdt[3];     // h / dt per dimension (Esirkepov)
     float norm;       // 1 / V
     int mask_words;
+    FlatLevels flat;
 };
 
 // all arguments of one ensemble's particle step (one kernel argument, or one entry of a batch)
@@ -442,7 +444,7 @@ __device__ __forceinline__ void particles_split_sc(const SplitArgs& A, long s)
         dts[d] = nn[d] + (PICA_CIC ? 3 : 4);
         dbase[d] = PICA_CIC ? m0[d] + 1 : m0[d];
     }
-    const TileStrides ts = tile_strides(NC == 4, NC == 0 && eg.ncps[2] == 1 ? eg.ncps[1] : 0, its, dts);
+    const TileStrides ts = tile_strides(NC == 4, NC == 0 ? sp.flat : FlatLevels{0, 0}, nn[1], its, dts);
     const int isx = ts.isx, isy = ts.isy, itn = ts.itn;
     const int dsx = ts.dsx, dsy = ts.dsy, dtn = ts.dtn;
     // every LDS pointer is smem + a byte offset, so that the compiler keeps DS instructions
@@ -1291,14 +1293,14 @@ __global__ void __launch_bounds__(PK_BLOCK) k_esk_sorted(GridView<float> g, EnsG
 }
 
 // dynamic LDS of k_particles_split (c4: its form for 4^3 supercells): field tile, FP64 J tile, mover mask, counters, mask prefix
-size_t split_lds(const pk_ens* e, bool c4, int shape, int dep, int mask_words)
+size_t split_lds(const pk_ens* e, bool c4, int shape, int dep, int mask_words, FlatLevels flat)
 {
     int its[3], dts[3];
     for (int d = 0; d < 3; d++) {
         its[d] = e->ncps[d] + (shape == PK_TSC ? 3 : 2);
         dts[d] = e->ncps[d] + ((shape == PK_CIC && dep == PK_DIRECT) ? 3 : 4);
     }
-    const TileStrides t = tile_strides(c4, e->ncps[2] == 1 ? e->ncps[1] : 0, its, dts);
+    const TileStrides t = tile_strides(c4, flat, e->ncps[1], its, dts);
     const size_t joff = (sizeof(float) * t.ni + 7) & ~(size_t)7;
     const size_t base = joff + sizeof(double) * t.nj + sizeof(uint64_t) * mask_words + sizeof(int) * 32 +
                         sizeof(long) * (mask_words + 1);
@@ -1324,7 +1326,8 @@ SplitArgs split_args(pk_ens* e, pk_grid* g, const EnsGeom& eg, const SplitParams
     return A;
 }
 
-int split_params(pk_ens* e, double dt, SplitParams& sp)
+// threads: of a workgroup
+int split_params(pk_ens* e, double dt, int shape, int dep, int threads, SplitParams& sp)
 {
     const double q = e->ctx->charge[e->type], m = e->ctx->mass[e->type];
     sp.coeff = (float)(q * dt / (2.0 * m * PK_C));
@@ -1337,6 +1340,10 @@ int split_params(pk_ens* e, double dt, SplitParams& sp)
     }
     sp.norm = (float)(1.0 / (e->step[0] * e->step[1] * e->step[2]));
     sp.mask_words = (e->maxcap + PK_BLOCK + 63) / 64 + 1;
+    sp.flat = FlatLevels{0, 0};
+    if (e->ncps[2] == 1)
+        sp.flat = pk_flat_levels([&](FlatLevels f) { return split_lds(e, false, shape, dep, sp.mask_words, f); },
+                                 20 * 64 / threads, shape == PK_TSC);
     return PK_OK;
 }
 
@@ -1345,8 +1352,8 @@ int launch(pk_ens* e, pk_grid* g, double dt)
 {
     EnsGeom eg = ens_geom(e);
     SplitParams sp;
-    if (int r = split_params(e, dt, sp)) return r;
-    const size_t lds = split_lds(e, NC == 4, SHAPE, DEP, sp.mask_words);
+    if (int r = split_params(e, dt, SHAPE, DEP, PK_BLOCK, sp)) return r;
+    const size_t lds = split_lds(e, NC == 4, SHAPE, DEP, sp.mask_words, sp.flat);
     if (lds > 160 * 1024) return pk_fail(e->ctx, PK_E_CAPACITY, "particle step: supercell too large for LDS");
     const unsigned nblocks = (unsigned)(PK_XCD * (long)eg.xcd_chunk);
     pk_ktimer tm(e->ctx, "particles");
@@ -1382,7 +1389,7 @@ int launch_sorted(pk_ens* e, pk_grid* g, double dt, const SortedLayout<SHAPE, NC
 {
     EnsGeom eg = ens_geom(e);
     SplitParams sp;
-    if (int r = split_params(e, dt, sp)) return r;
+    if (int r = split_params(e, dt, SHAPE, PK_ESIRKEPOV, PK_BLOCK, sp)) return r;
     if (sp.mask_words != L.mask_words) return pk_fail(e->ctx, PK_E_STATE, "particle step: stale LDS layout");
     const unsigned nblocks = (unsigned)(PK_XCD * (long)eg.xcd_chunk);
     PK_HIP(e->ctx, hipFuncSetAttribute((const void*)k_esk_sorted<SHAPE, NC>,
@@ -1500,10 +1507,10 @@ int pk_batch_split_prepare(pk_batch* b, double dt, int shape, int dep)
     for (int i = 0; i < n; i++) {
         pk_ens* e = b->ens[i];
         SplitParams sp;
-        if (int r = split_params(e, dt, sp)) return r;
-        jobs[i] = split_args(e, b->grids[i], ens_geom(e), sp);
         const int sh = pk_batch_shape_of(b, i, shape);
-        const size_t l = split_lds(e, c4, sh, dep, sp.mask_words);
+        if (int r = split_params(e, dt, sh, dep, b->knob[PK_BATCH_BLOCK], sp)) return r;
+        jobs[i] = split_args(e, b->grids[i], ens_geom(e), sp);
+        const size_t l = split_lds(e, c4, sh, dep, sp.mask_words, sp.flat);
         if (l > b->cplds[sh]) b->cplds[sh] = l;
     }
     if (b->cplds[0] > 160 * 1024 || b->cplds[1] > 160 * 1024)
