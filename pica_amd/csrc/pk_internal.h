@@ -256,10 +256,11 @@ __device__ __forceinline__ int pk_select_bit(uint64_t m, int k)
 // by one wavefront: pre[w] = set bits of mask[0 .. w), w <= words.  Up to FEW words each lane counts those below its
 // own; more go 64 at a time, through six dependent
 // shuffles, which a supercell of 16 particles feels (504 x 504 x 16 ppc in supercells of one cell, FP32 CIC direct:
-// 2152 us with shuffles, 2063 us so, 2053 us by one lane, which a full supercell waits for).
+// 2137-2152 us with shuffles, 2063-2087 us so, 2053 us by one lane, which a full supercell waits for).  FEW = 8
+// costs the batched FP32 step 3% (64 plasmas, TSC direct: 635 us a step, 615 us with 4) and gains nothing.
 __device__ __forceinline__ void pk_mask_prefix(const uint64_t* mask, long* pre, int words, int lane)
 {
-    constexpr int FEW = 8;
+    constexpr int FEW = 4;
     int run = 0;
     if (words <= FEW) {
 #pragma unroll

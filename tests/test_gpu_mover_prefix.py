@@ -1,5 +1,5 @@
 """The order of a supercell's movers and of the holes they leave, by the count of its particles: one mask word, the
-most that each lane counts by itself (8 words of 64) and one more, and more than 64 words, against the oracle.
+most that each lane counts by itself (4 words of 64) and one more, and more than 64 words, against the oracle.
 
 FP64: order bit-exact, every field within 1e-12 of the oracle's after 3 steps; FP32: the same set of particles and the
 split form's bounds.
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("prec", [P.F64, P.F32])
-@pytest.mark.parametrize("n", [1, 64, 65, 128, 129, 449, 512, 513, 576, 4096, 4097])
+@pytest.mark.parametrize("n", [1, 64, 65, 128, 129, 192, 255, 256, 257, 321, 449, 512, 513, 576, 4096, 4097])
 def test_movers_of_one_supercell(ctx, prec, n):
     _say("mover prefix prec=%d n=%d" % (prec, n))
     rng = np.random.default_rng(n)
