@@ -551,9 +551,11 @@ __global__ void __launch_bounds__(PK_BLOCK) k_particles(GridView<double> g, EnsG
 #include "pk_particles_f64_body.inc"
 }
 
-// many ensembles: a list of (ensemble, supercell) items; gridDim.x < nitems makes it persistent
+// many ensembles: a list of (ensemble, supercell) items; gridDim.x < nitems makes it persistent.  At least three
+// wavefronts a SIMD with Esirkepov: the compiler takes 176 VGPRs for TSC otherwise, and two (64 plasmas of 16^3 to
+// 32^3 cells at 4 and 8 ppc, a step: 1049 us with two, 877 us with three, which need no spill)
 template <int SHAPE, int DEP, int NC>
-__global__ void __launch_bounds__(PK_BLOCK) k_particles_batch(const F64Args* __restrict__ jobs,
+__global__ void __launch_bounds__(PK_BLOCK, DEP == PK_ESIRKEPOV ? 3 : 1) k_particles_batch(const F64Args* __restrict__ jobs,
                                                               const int2* __restrict__ items, long nitems,
                                                               const int* __restrict__ halt)
 {
