@@ -128,6 +128,7 @@ int pk_ctx_create(int device, pk_ctx** out)
         hipHostMalloc((void**)&c->flags_host, sizeof(int32_t) * PK_NFLAGS, hipHostMallocDefault) != hipSuccess ||
         hipEventCreateWithFlags(&c->flags_ev, hipEventDisableTiming) != hipSuccess ||
         !(c->staging = pk_staging_create())) {
+        if (c->flags_ev) (void)hipEventDestroy(c->flags_ev);
         if (c->flags_host) (void)hipHostFree(c->flags_host);
         if (c->stream) (void)hipStreamDestroy(c->stream);
         delete c;
