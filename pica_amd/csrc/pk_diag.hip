@@ -13,10 +13,13 @@ constexpr int NR = 7;               // grid reduction slots
 
 // rho of one supercell's particles into an LDS tile (cell-centre nodes, base m+1, n+2 wide),
 // flushed x 1/V with FP64 atomics.  Shape weights as the oracle's or_deposit_rho.  The LDS atomics bound it
-// (27 a particle with TSC, ~9 cycles of a CU each): an FP32 lane takes two adjacent slots, which the
-// interleave fills from one cell, and adds both with one set; 4^3 supercells have rows of 12 doubles, so
-// that the 16 cells of an x plane meet 16 LDS bank pairs.  96^3 x 8 ppc, FP32 TSC: 50 us against 117.
-constexpr int RHO_SY4 = 12;
+// (27 a particle with TSC, ~9 cycles of a CU each): where cells hold two particles or more on average, an FP32 lane
+// takes two adjacent slots, which the interleave fills from one cell, and adds both with one set; 4^3 supercells have
+// rows of 12 doubles, so that the 16 cells of an x plane meet 16 LDS bank pairs.  96^3 x 8 ppc, FP32 TSC: 50 us against
+// 117.  Fewer than RHO_SHARE pairs of a wavefront that share their nodes are added one by one: their own set of
+// atomics would come on top of the others' two (64^3 x 33 ppc never interleaved, with fold and fill: 241 us, 253 us
+// with every such pair added together, 235 us one particle a lane; right after an interleave 83, 83 and 162 us).
+constexpr int RHO_SY4 = 12, RHO_SHARE = 16;
 template <int SHAPE, bool SPLIT, int NC>
 __global__ void __launch_bounds__(256) k_rho(EnsGeom eg, PartF64 pf, PartSplit ps, const int64_t* off,
                                              const int32_t* cnt, double q, double* rho, int s1, int s2)
@@ -89,12 +92,14 @@ __global__ void __launch_bounds__(256) k_rho(EnsGeom eg, PartF64 pf, PartSplit p
                 for (int c = 0; c < K; c++)
                     atomicAdd(&tile[A.at + a * sx + bb * sy + c], A.wt[0][a] * A.wt[1][bb] * A.wt[2][c] * A.qw);
     };
-    if (SPLIT) {
+    if (SPLIT && n >= 2 * eg.ncps[0] * eg.ncps[1] * eg.ncps[2]) {
         for (int l = 2 * threadIdx.x; l < n; l += 2 * blockDim.x) {
             Term A, B;
             term(l, A);
             term(l + 1, B);
-            if (A.ok && B.ok && A.at == B.at) {
+            bool same = A.ok && B.ok && A.at == B.at;
+            if (__popcll(__ballot(same)) < RHO_SHARE) same = false;
+            if (same) {
 #pragma unroll
                 for (int a = 0; a < K; a++)
 #pragma unroll
