@@ -108,7 +108,11 @@ int pk_species_set(pk_ctx* ctx, int ntypes, const double* mass, const double* ch
 int pk_grid_create(pk_ctx* ctx, int prec, const int size[3], const double origin[3], const double step[3],
                    int ghost, pk_grid** out);
 void pk_grid_destroy(pk_grid* g);
-/* copy one component (PK_EX..PK_RHO) between host and device; host element type = grid prec */
+/* copy one component (PK_EX..PK_RHO) between host and device; host element type = grid prec.
+ * Copies of 1 MB and more to host memory that the device cannot reach (here and in
+ * pk_ens_download) go through pinned memory of the context: 1 to 8 MB, allocated by the first such
+ * copy (which takes up to 1.5 ms longer in the first contexts of a process), used by one copy at a
+ * time, freed with the context; above 6 MB three host threads help with the copy. */
 int pk_grid_copy(pk_grid* g, int comp, void* host, int dir);
 int pk_grid_zero(pk_grid* g, int comp);
 /* YeeSolver::updateE / updateB (YeeSolver.h:14-18,132-213): pica's semantics on the whole

@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(256) k_yee_b(GridView<T> g, YeeCoef<T> k, long
 // cells, G <= PK_MAX_PERIODIC_GHOST ghost layers a side), -1 if it is none: c = 0 is p itself, then the
 // low ghosts, then the high ghosts, ascending.  M = 1 + 2 G of them in general; with n >= 2 G a cell has
 // one ghost at most, and M = 2.  Computed and not listed in an array: an array indexed at run time lives in
-// scratch memory (fold and fill of J on 20^3 nodes took 7.8 + 4.8 us with lists, in two launches).
+// scratch memory (fold and fill of J of 32^3 FP64 cells took 7.8 + 4.7 us with lists, in two launches; 4.2 us now).
 constexpr int MAX_IMAGES = 1 + 2 * PK_MAX_PERIODIC_GHOST;
 template <int M>
 __device__ __forceinline__ int image_at(int c, int p, int n, int G)
@@ -199,7 +199,7 @@ __global__ void __launch_bounds__(256) k_yee_b_periodic(GridView<T> g, YeeCoef<T
 // value is that fold's bit for bit, and (fill) writes it back into them.  A ghost images one cell, so no
 // other thread reads what this one writes.  Without fill the ghosts keep their values (the caller reads
 // only physical cells until it fills them); a cell with no image along any dimension is left alone.
-// 128^3 FP64: 11.6 + 7.8 us in two launches before.
+// FP64, us, in two launches before and now: 128^3 10.6 + 7.7, 8.2; 256^3 24.9 + 15.2, 27.2.
 // the physical cells within G of a face, each once: slab x (i near a face; any j, k), then slab y
 // (i inside; j near a face), then slab z (i, j inside; k near a face).  nb = cells near a face
 // along a dimension (all n when n <= 2G)

@@ -213,8 +213,8 @@ struct FlatLevels {
     int field, j;
 };
 
-// The levels of a supercell's field and J tiles.  lds(levels): bytes of a workgroup; most: workgroups a CU that the
-// registers allow; even: the field tile's rows are even (TSC).  The highest levels that leave as many workgroups on a
+// The levels of a supercell's field and J tiles.  lds(levels): bytes of a workgroup; most: workgroups a CU beyond which
+// more bring nothing; even: the field tile's rows are even (TSC).  The highest levels that leave as many workgroups on a
 // CU as level 0 does, J first (its atomics cost more than reads), since a workgroup less costs more than the conflicts:
 // 504 x 504 x 16 ppc, us a step at level 0 / level 2 whatever the LDS / now: FP32 CIC Esirkepov 12 x 4 cells 207 / 226 /
 // 170, FP64 CIC direct 12 x 12 234 / 241 / 233, FP64 TSC direct 12 x 12 551 / 623 / 519.  Even rows of the field tile

@@ -13,9 +13,12 @@
 //      class), and the stayers found past the final count fill the holes movers left below it
 //      (ascending order on both sides);
 //   4. flush the J tile x 1/V with one pass of global FP64 atomics (the destructor, :201-213).
-// This file is compiled with -ffp-contract=off: per particle, the arithmetic is pica's, in
-// pica's order, so positions and momenta agree with pica to the last bit given the same
-// fields.  The only FP difference left is the order of J sums (atomics).
+// This file is compiled with -ffp-contract=off: interpolation, push and direct deposition are pica's
+// arithmetic in pica's order, so positions and momenta agree with pica to the last bit given the same
+// fields, and a particle's direct currents do; the order in which they are summed into J (atomics) is
+// free.  Esirkepov's currents, which pica does not have, are rounded as esk_stay, esk_change and
+// esk_window below evaluate them (nearer to the exact ones than the sum over old and new shape: of a
+// staying TSC particle 1.3e-16 of its currents against 2.8e-15, of a CIC one 8e-17 against 1.2e-16).
 #include "pk_internal.h"
 
 namespace {

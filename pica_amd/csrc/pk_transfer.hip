@@ -1,10 +1,12 @@
 // pk_transfer.hip -- device memory to ordinary host memory.
 //
-// The runtime copies to pageable memory at 16 GB/s at best: into freshly mapped destinations on MI355X 311 us for
-// 4.2 MB, 560 us for 9.2 MB, 1104 us for 18.4 MB, 6.7 ms for 70 MB.  Here a small kernel writes the bytes into pinned
-// memory chunk by chunk (the link takes 50 GB/s), and host threads move each chunk on while the next ones are under
-// way: 139, 245 and 441 us and 2.3 ms for the same sizes.  What bounds it is the host's first touch of fresh
-// destination pages, hence the extra threads for large copies.
+// The runtime copies to pageable memory at 18 GB/s at best: on MI355X 250 us for 4.2 MB, 510 us for 9.2 MB, 1020 us
+// for 18.4 MB and 3.9 ms for 70 MB into pages in use, 680 us, 1.25 ms, 2.0 ms and 7.8 ms into fresh ones.  Here a
+// small kernel writes the bytes into pinned memory chunk by chunk (the link takes 50 GB/s), and host threads move
+// each chunk on while the next ones are under way: 140, 250 and 450 us and 1.6 ms into pages in use, 490, 530 and
+// 800 us and 2.5 ms into fresh ones.  What bounds it there is the host's first touch, hence the extra threads for
+// large copies.  The pinned memory is allocated by the first copy that needs it: 1 to 1.5 ms in the first contexts
+// of a process, 0.1 ms later.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -24,8 +26,8 @@ constexpr int HELPERS = 3;       // host threads besides the caller; one more br
 // up to here the caller alone keeps up (4 MB: 138 us alone in 512 KB chunks, 141 us with helpers in 1 MB ones;
 // 9.2 MB: 306 against 245 us)
 constexpr size_t ALONE = 6 << 20;
-// below this the runtime's copy is as fast (187 KB: 17 us against 19 here; 1 MB: 68 against 73 us where the
-// destination is in use already, 450 against 50 us where it is fresh)
+// below this the runtime's copy is as fast (187 KB, 373 KB, 953 KB: 18, 25 and 50 us against 20, 28 and 50 here into
+// pages in use, 19, 74 and 175 against 23, 78 and 182 into fresh ones; 1.1 MB: 72 against 52 and 260 against 200)
 constexpr size_t DIRECT = 1 << 20;
 
 template <class V>
