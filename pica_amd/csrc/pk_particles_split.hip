@@ -320,15 +320,13 @@ __device__ __forceinline__ void esk_stay_shapes(const float o[3], const float on
     for (int d = 0; d < 3; d++) {
         const float s0 = o[d] - 0.5f, s1 = on[d] - 0.5f;
         if (SHAPE == PK_TSC) {
-            float w0[3], w1[3];
-            tsc_w(s0, w0);
-            tsc_w(s1, w1);
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                asm("" : "+v"(w1[k]));      // rounded before the difference, as in esk_shapes
-                S0[d][k] = w0[k];
-                DS[d][k] = w1[k] - w0[k];
-            }
+            const float a0 = 0.5f - s0, b0 = 0.5f + s0, a1 = 0.5f - s1, b1 = 0.5f + s1;
+            S0[d][0] = 0.5f * a0 * a0;
+            S0[d][1] = fmaf(-s0, s0, 0.75f);
+            S0[d][K - 1] = 0.5f * b0 * b0;
+            DS[d][0] = fmaf(-0.5f * a0, a0, 0.5f * a1 * a1);
+            DS[d][1] = fmaf(-s1, s1, 0.75f) - S0[d][1];
+            DS[d][K - 1] = fmaf(-0.5f * b0, b0, 0.5f * b1 * b1);
         } else {
             const float f0 = s0 < 0.0f ? s0 + 1.0f : s0, f1 = s1 < 0.0f ? s1 + 1.0f : s1;
             S0[d][0] = 1.0f - f0;
@@ -341,7 +339,9 @@ __device__ __forceinline__ void esk_stay_shapes(const float o[3], const float on
 
 // Esirkepov deposit of a staying particle P, or (PAIR) of two on one K x K x K window: every tile
 // node receives the sum of both particles' terms with one atomic.  qwQ = 0 (and finite offsets of Q)
-// deposits P alone.
+// deposits P alone.  Here and in esk_stay_shapes the products that are not rounded are written out: which of two
+// the compiler fuses depends on the code around them, and another choice moves the last bit of J by up to 1e-7,
+// which the BF16 network of a denoised step turns into 1e-4 of its fields.
 template <int SHAPE, bool PAIR>
 __device__ __forceinline__ void esk_stay(double* jt, int dtn, int sx, int sy, const int w[3], const float oP[3],
                                          const float onP[3], float qwP, const float oQ[3], const float onQ[3], float qwQ,
@@ -361,16 +361,19 @@ __device__ __forceinline__ void esk_stay(double* jt, int dtn, int sx, int sy, co
         double* t = jt + comp * dtn + orig + st[comp];
 #pragma unroll
         for (int p = 0; p < K; p++) {
-            const float AP = kP * (S0P[d1][p] + 0.5f * DSP[d1][p]), BP = kP * (0.5f * S0P[d1][p] + third * DSP[d1][p]);
-            const float AQ = kQ * (S0Q[d1][p] + 0.5f * DSQ[d1][p]), BQ = kQ * (0.5f * S0Q[d1][p] + third * DSQ[d1][p]);
+            const float AP = kP * fmaf(0.5f, DSP[d1][p], S0P[d1][p]), BP = kP * fmaf(third, DSP[d1][p], 0.5f * S0P[d1][p]);
+            const float AQ = kQ * fmaf(0.5f, DSQ[d1][p], S0Q[d1][p]), BQ = kQ * fmaf(third, DSQ[d1][p], 0.5f * S0Q[d1][p]);
 #pragma unroll
             for (int r = 0; r < K; r++) {
-                const float cp = AP * S0P[d2][r] + BP * DSP[d2][r];
-                const float cq = AQ * S0Q[d2][r] + BQ * DSQ[d2][r];
+                const float cp = comp == 1 ? fmaf(BP, DSP[d2][r], AP * S0P[d2][r]) : fmaf(AP, S0P[d2][r], BP * DSP[d2][r]);
+                const float cq = comp == 1 ? fmaf(BQ, DSQ[d2][r], AQ * S0Q[d2][r]) : fmaf(AQ, S0Q[d2][r], BQ * DSQ[d2][r]);
                 float cum = 0.0f;
 #pragma unroll
                 for (int a = 0; a < K - 1; a++) {
-                    cum += PAIR ? DSP[comp][a] * cp + DSQ[comp][a] * cq : DSP[comp][a] * cp;
+                    if (PAIR)
+                        cum += fmaf(DSQ[comp][a], cq, DSP[comp][a] * cp);
+                    else
+                        cum = fmaf(DSP[comp][a], cp, cum);
                     atomicAdd(&t[a * st[comp] + p * st[d1] + r * st[d2]], (double)cum);
                 }
             }
